@@ -12,9 +12,10 @@
 // Q4_0 nibbles expanded to signed int8 q-8), with a 16-byte row pad against bank conflicts. Tiles
 // are numbered so that the workgroups sharing one weight tile land on the same XCD (and L2).
 //
-// The per-block epilogue (3 VALU operations per output element per K-block of 32, against one
-// 32-deep MFMA step) bounds this kernel near 1/6 of the int8 MFMA peak: ggml's semantics put a
-// scale on every block, so the block sums cannot stay in the int32 accumulator.
+// The per-block epilogue (2 VALU operations per output element per K-block of 32, against one
+// 32-deep MFMA step) bounds this kernel: ggml's semantics put a scale on every block, so the block
+// sums cannot stay in the int32 accumulator. With a conversion as a third operation Q8_0 512 x 14336
+// x 4096 took 114.8 us with the activation's quantization; taken out by the start value below, 104.0 us.
 #include "gcq_common.h"
 
 namespace gcq {
@@ -25,6 +26,13 @@ typedef int v16i __attribute__((ext_vector_type(16)));
 constexpr int GBM = 128, GBN = 128;  // workgroup tile
 constexpr int GKB = 2;               // K-blocks (of 32) per LDS stage
 constexpr int GPITCH = GKB * 32 + 16;  // LDS row pitch in bytes (16 B pad against bank conflicts)
+
+// The MFMAs start from the bits of 1.5 * 2^23 instead of 0, so an int32 block sum (|isum| < 2^22) comes
+// out as the bits of the float 1.5 * 2^23 + isum: no conversion. d_w is an fp16 value, so
+// fma(that, d_w, -1.5 * 2^23 d_w) has an exact product and an exact constant: one rounding, of
+// isum * d_w, the same float that converting and multiplying gives.
+constexpr int kMagicBits = 0x4B400000;
+constexpr float kMagic = 12582912.0f;
 
 __device__ __forceinline__ uint32_t q4_to_s8(uint32_t w) {  // 4 nibbles (0..15) -> 4 int8 (q - 8)
     return (((w & 0x0F0F0F0Fu) | 0x80808080u) - 0x08080808u) ^ 0x80808080u;
@@ -138,7 +146,7 @@ __device__ __forceinline__ void gemm_store(const GemmStage<TYPE> & st, int8_t * 
 //
 // Pipeline: chunk c + 1's global loads are issued into registers before chunk c is computed from
 // LDS, then stored to the other LDS buffer; one barrier per chunk. Per K-block each wavefront
-// issues its four 32x32x32 MFMAs, then folds each int32 result into the fp32 accumulators as
+// issues its four 32x32x32 MFMAs, then folds each block sum into the fp32 accumulators as
 // (isum * d_w) * d_x, the scales read from LDS once per block as vectors.
 template <int TYPE, bool RAW>
 __global__ __launch_bounds__(256) void k_gemm(const uint8_t * __restrict__ wqs, const uint16_t * __restrict__ wd,
@@ -167,6 +175,11 @@ __global__ __launch_bounds__(256) void k_gemm(const uint8_t * __restrict__ wqs, 
         for (int b = 0; b < 2; b++)
 #pragma unroll
             for (int r = 0; r < 16; r++) acc[a][b][r] = 0.0f;
+
+    v16i magic;
+#pragma unroll
+    for (int r = 0; r < 16; r++) magic[r] = kMagicBits;
+    asm volatile("" : "+v"(magic));  // kept in registers: known constants are written again before every block
 
     const int kb_begin = RAW ? raw_blk : 0;
     const int kb_end = RAW ? raw_blk + 1 : nb;
@@ -197,14 +210,14 @@ __global__ __launch_bounds__(256) void k_gemm(const uint8_t * __restrict__ wqs, 
             for (int tm = 0; tm < 2; tm++)
 #pragma unroll
                 for (int tn = 0; tn < 2; tn++)
-                    cc[tm][tn] = __builtin_amdgcn_mfma_i32_32x32x32_i8(af[tm], bf[tn], v16i{}, 0, 0, 0);
+                    cc[tm][tn] = __builtin_amdgcn_mfma_i32_32x32x32_i8(af[tm], bf[tn], magic, 0, 0, 0);
             if constexpr (RAW) {
 #pragma unroll
                 for (int tm = 0; tm < 2; tm++)
 #pragma unroll
                     for (int tn = 0; tn < 2; tn++)
 #pragma unroll
-                        for (int r = 0; r < 16; r++) acc[tm][tn][r] = __int_as_float(cc[tm][tn][r]);
+                        for (int r = 0; r < 16; r++) acc[tm][tn][r] = __int_as_float(cc[tm][tn][r] - kMagicBits);
             } else {
                 // d_x of this lane's rows: element r of tile tm is row wm*64 + tm*32 + 8*(r/4) + 4*(lane/32) + r%4
                 float4 dx[2][4];
@@ -214,19 +227,33 @@ __global__ __launch_bounds__(256) void k_gemm(const uint8_t * __restrict__ wqs, 
                     for (int q = 0; q < 4; q++)
                         dx[tm][q] = *reinterpret_cast<const float4 *>(sdx[buf] + j * GBM + wm * 64 + tm * 32 + q * 8 +
                                                                       (lane >> 5) * 4);
-                float dwv[2];
+                float dwv[2], cw[2];
 #pragma unroll
-                for (int tn = 0; tn < 2; tn++) dwv[tn] = sdw[buf][j * GBN + wn * 64 + tn * 32 + (lane & 31)];
+                for (int tn = 0; tn < 2; tn++) {
+                    dwv[tn] = sdw[buf][j * GBN + wn * 64 + tn * 32 + (lane & 31)];
+                    cw[tn] = -kMagic * dwv[tn];
+                }
+                if (__builtin_expect(__any(__builtin_isinf(dwv[0]) || __builtin_isinf(dwv[1])), 0)) {
+                    // an infinite weight scale: isum * inf, which inf - inf would make a NaN
+#pragma unroll
+                    for (int tm = 0; tm < 2; tm++)
+#pragma unroll
+                        for (int tn = 0; tn < 2; tn++)
+#pragma unroll
+                            for (int r = 0; r < 16; r++)
+                                cc[tm][tn][r] = __float_as_int(__int_as_float(cc[tm][tn][r]) - kMagic);
+                    cw[0] = cw[1] = 0.0f;
+                }
 #pragma unroll
                 for (int tm = 0; tm < 2; tm++)
 #pragma unroll
                     for (int tn = 0; tn < 2; tn++)
 #pragma unroll
                         for (int q = 0; q < 4; q++) {
-                            acc[tm][tn][4 * q + 0] += ((float) cc[tm][tn][4 * q + 0] * dwv[tn]) * dx[tm][q].x;
-                            acc[tm][tn][4 * q + 1] += ((float) cc[tm][tn][4 * q + 1] * dwv[tn]) * dx[tm][q].y;
-                            acc[tm][tn][4 * q + 2] += ((float) cc[tm][tn][4 * q + 2] * dwv[tn]) * dx[tm][q].z;
-                            acc[tm][tn][4 * q + 3] += ((float) cc[tm][tn][4 * q + 3] * dwv[tn]) * dx[tm][q].w;
+                            acc[tm][tn][4 * q + 0] = fmaf(fmaf(__int_as_float(cc[tm][tn][4 * q + 0]), dwv[tn], cw[tn]), dx[tm][q].x, acc[tm][tn][4 * q + 0]);
+                            acc[tm][tn][4 * q + 1] = fmaf(fmaf(__int_as_float(cc[tm][tn][4 * q + 1]), dwv[tn], cw[tn]), dx[tm][q].y, acc[tm][tn][4 * q + 1]);
+                            acc[tm][tn][4 * q + 2] = fmaf(fmaf(__int_as_float(cc[tm][tn][4 * q + 2]), dwv[tn], cw[tn]), dx[tm][q].z, acc[tm][tn][4 * q + 2]);
+                            acc[tm][tn][4 * q + 3] = fmaf(fmaf(__int_as_float(cc[tm][tn][4 * q + 3]), dwv[tn], cw[tn]), dx[tm][q].w, acc[tm][tn][4 * q + 3]);
                         }
             }
         }
