@@ -9,19 +9,29 @@
 //                8 sub-blocks of 32; y += d_x(m) (d_w(n) I1 - dmin_w(n) I2)
 //   Q6_K:        I1 = sum_j sc_j(n) isum_j(m, n) over the 16 sub-blocks of 16 (codes q - 32);
 //                y += d_x(m) d_w(n) I1
-// isum_j is one MFMA: v_mfma_i32_32x32x32_i8 over a 32-value sub-block, v_mfma_i32_32x32x16_i8 over
-// a 16-value one. I1 takes the sub-block's 6-bit / int8 scale on the VALU (one integer
-// multiply-add per output and sub-block). I2 is itself a small integer product over the 8
-// sub-blocks: the activation's block sums split into bytes (bs = 64 hi + lo, lo in [0, 64)) against
-// the weight's 6-bit mins, two MFMAs of K 32 (8 used) per super-block.
 //
-// Workgroup tile 128 (m) x 128 (n), 8 wavefronts of 64 x 32 (2 MFMA tiles of 32 x 32). The K
-// loop steps half a super-block (128 values) at a time: the next half's global loads are issued
-// into registers before the current half is computed from LDS, then stored (weights expanded to
-// int8 codes, the super-block's scales decoded); activations and weights of a tile are read once
-// per workgroup. A wavefront's 64 outputs per lane (f32 sums and the super-block's int32 sums) keep it
-// within 256 registers, two wavefronts per SIMD. Tiles are numbered
-// so that the workgroups sharing a weight tile land on one XCD.
+// The sub-block scales go into the weight operand, so I1 is formed by the matrix cores alone: a
+// weight enters as two int8 codes, hi and lo, with I1 = S sum(hi x) + sum(lo x) over the whole
+// super-block in two int32 accumulators (v_mfma_i32_32x32x32_i8, twice the MFMAs of the bare codes).
+//   Q4_K: sc = 8 sh + sl (sh, sl < 8): hi = sh q, lo = sl q (<= 105), S = 8
+//   Q5_K: the same with q <= 31 (products <= 217 fit a byte but not an int8): taken minus 128, and both
+//         accumulators start from 128 times the row's code sum of the super-block
+//   Q6_K: v = sc (q - 32) in [-4096, 4096]: hi = v >> 6, lo = v & 63, S = 64
+// I2 is one f16 MFMA of K 16 per tile and super-block: the activation's block sums in two f16 parts
+// (a multiple of 64 and the rest) against the 6-bit mins, exact in f32.
+//
+// A workgroup is KG K groups of WN wavefronts; a wavefront takes 32 XT rows (m) x 32 columns (n), its tile
+// 32 XT x 32 WN. Group g takes the super-blocks g, g + KG, ...; the groups' sums meet in LDS at the end
+// (more wavefronts where the tiles are few). The activation codes go through LDS, double-buffered
+// in steps of half a super-block (rows of 128 B at a pitch of 144 B: 8 lanes' 16-byte reads fall in
+// distinct banks). So do the weights, as they are in memory (loaded in whole rows, 5 KB a step):
+// lane (column, k half) reads its column's 16-byte pieces and expands them to hi and lo codes right
+// where the MFMA takes them, its column's header (scales, mins, d) in its own registers.
+//
+// What bounds it: the VALU's issue (about 190 operations per wavefront and half super-block beside 16
+// MFMAs: the expansion, then 5 operations per output and super-block). Measured, the GEMM alone
+// at Q4_K 1999 x 14336 x 4096: 435 us with the sub-block scales applied on the VALU (an integer
+// multiply-add per output and 32 values), 340 us as here; 33 x 4096 x 14336 (KG = 8): 133 -> 21 us.
 #include "gcq_common.h"
 
 namespace gcq {
@@ -32,51 +42,24 @@ namespace {
 
 typedef int v4i __attribute__((ext_vector_type(4)));
 typedef int v16i __attribute__((ext_vector_type(16)));
+typedef float v16f __attribute__((ext_vector_type(16)));
+typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
+typedef int16_t i16x2 __attribute__((ext_vector_type(2)));
+typedef _Float16 h2_t __attribute__((ext_vector_type(2)));
+typedef _Float16 h4_t __attribute__((ext_vector_type(4)));
+typedef _Float16 h8_t __attribute__((ext_vector_type(8)));
 
-constexpr int TM = 128;            // workgroup tile rows; its columns TN: 128, or 64 for small grids
-constexpr int NT = 512;            // threads: 8 wavefronts of 64 (m) x 32 (n)
-constexpr int HV = 128;            // values per K step (half a super-block)
-constexpr int KP = HV + 16;        // LDS row pitch of the codes (bytes; 16 B pad against bank conflicts)
+// LDS row pitches (bytes) of half a super-block's codes, low bits and high bits: 8 lanes' 16-byte reads
+// of consecutive rows fall in distinct banks.
+constexpr int KP = 128 + 16, WP = 64 + 16, QP = 32 + 16;
 
 template <int TYPE>
 struct Kq {
-    static constexpr int BB = 128;  // the low bits' bytes per super-block (nibbles / Q6_K's ql)
-    static constexpr bool MIN = TYPE != T_Q6_K;  // a min term (Q4_K / Q5_K)
-    static constexpr int NSUB = TYPE == T_Q6_K ? 16 : 8;  // scales per super-block
+    static constexpr bool MIN = TYPE != T_Q6_K;   // a min term (Q4_K / Q5_K)
+    static constexpr bool BIAS = TYPE == T_Q5_K;  // operand bytes taken minus 128
+    static constexpr int QH = TYPE == T_Q6_K ? 64 : 32;  // high-bit bytes per super-block
 };
 
-// Registers between one K step's global loads and its LDS store (thread t's share).
-template <int TYPE>
-struct KqStage {
-    v4i a[2];          // activation codes: 128 rows x 128 B, 16 B chunks t and t + 512
-    v4i b;             // weight bytes: Q4_K / Q5_K 16 B of nibbles; Q6_K (t < 256) ql, first half
-    v4i b2;            // Q5_K: 16 B of qh; Q6_K: ql, second half
-    v4i b3;            // Q6_K: 16 B of qh
-    // first half only: t < 128: e0 = the weight row's 16 B of d / dmin / scales (Q6_K: scales),
-    // dw = its fp16 d (Q6_K); t >= 128: e0, e1 = the activation row's 16 block sums (int16), dx
-    // its d. (One pair of registers for both: loads into different members on the two sides of
-    // a branch became one load into a private-memory slot picked by the branch.)
-    v4i e0, e1;
-    uint32_t dw;
-    float dx;
-};
-
-__device__ __forceinline__ uint32_t u32(int x) { return (uint32_t) x; }
-
-// 6-bit (scale, min) of sub-block j from ggml's 12 packed bytes (get_scale_min_k4), the bytes
-// held 4 per word in w[0..2] (register values: no byte pointer into them).
-__device__ __forceinline__ int sbyte(const uint32_t (&w)[3], int k) { return (int) ((w[k >> 2] >> (8 * (k & 3))) & 0xffu); }
-__device__ __forceinline__ void scale_min(const uint32_t (&q)[3], int j, int & sc, int & m) {
-    if (j < 4) {
-        sc = sbyte(q, j) & 63;
-        m = sbyte(q, j + 4) & 63;
-    } else {
-        sc = (sbyte(q, j + 4) & 0xF) | ((sbyte(q, j - 4) >> 6) << 4);
-        m = (sbyte(q, j + 4) >> 4) | ((sbyte(q, j) >> 6) << 4);
-    }
-}
-
-template <int TYPE>
 struct KqArgs {
     const uint8_t * w;      // packed weight's low bits: [N][nsb][128] (nibbles / Q6_K's ql)
     const uint16_t * wd;    // Q6_K: fp16 d [N][nsb]
@@ -87,308 +70,361 @@ struct KqArgs {
     const float * xd;       // d [M][K / 256]
     float * y;
     const float * res;
-    int32_t * raw;          // RAW: the integer parts of super-block raw_sb, [M][N][2] (Q6_K: [M][N][1]), stored
-                            // when its second half is done
+    int32_t * raw;          // RAW: the integer parts of super-block raw_sb, [M][N][2] (Q6_K: [M][N][1])
     int M, N, nsb, ldy, raw_sb;
 };
 
-template <int TYPE, int TN>
-__device__ __forceinline__ void kq_load(KqStage<TYPE> & st, const KqArgs<TYPE> & a, int m0, int n0, int step) {
-    const int t = threadIdx.x;
-    const int sb = step >> 1, h = step & 1;
-    const int K = a.nsb * 256;
-#pragma unroll
-    for (int q = 0; q < 2; q++) {
-        const int c = t + NT * q, row = c >> 3, part = c & 7;
-        const int m = min(m0 + row, a.M - 1);
-        st.a[q] = *reinterpret_cast<const v4i *>(a.xc + (size_t) m * K + sb * 256 + h * HV + 16 * part);
-    }
-    if constexpr (TYPE == T_Q6_K) {
-        if (t < 2 * TN) {  // row t / 2, bytes l0 .. l0 + 15 of each 32 of the half
-            const int row = t >> 1, l0 = 16 * (t & 1);
-            const size_t bi = (size_t) min(n0 + row, a.N - 1) * a.nsb + sb;
-            const uint8_t * ql = a.w + bi * 128;
-            st.b = *reinterpret_cast<const v4i *>(ql + 64 * h + l0);
-            st.b2 = *reinterpret_cast<const v4i *>(ql + 64 * h + 32 + l0);
-            st.b3 = *reinterpret_cast<const v4i *>(a.wqh + bi * 64 + 32 * h + l0);
-        }
-    } else if (t < 4 * TN) {
-        // row t / 4, u = t % 4: 16 B of nibbles (and Q5_K the matching 16 B of qh)
-        const int row = t >> 2, u = t & 3;
-        const size_t bi = (size_t) min(n0 + row, a.N - 1) * a.nsb + sb;
-        st.b = *reinterpret_cast<const v4i *>(a.w + bi * 128 + 64 * h + 16 * u);
-        if constexpr (TYPE == T_Q5_K) st.b2 = *reinterpret_cast<const v4i *>(a.wqh + bi * 32 + 16 * (u & 1));
-    }
-    if (h == 0) {
-        if (t < TN) {
-            const size_t bi = (size_t) min(n0 + t, a.N - 1) * a.nsb + sb;
-            st.e0 = *reinterpret_cast<const v4i *>(a.whdr + bi * 16);  // header / Q6_K scales
-            if constexpr (TYPE == T_Q6_K) st.dw = a.wd[bi];
-        } else if (t < TN + TM) {
-            const int m = min(m0 + t - TN, a.M - 1);
-            st.dx = a.xd[(size_t) m * a.nsb + sb];
-            const v4i * bp = reinterpret_cast<const v4i *>(a.xbs + (size_t) m * (a.nsb * 16) + sb * 16);
-            st.e1 = bp[1];
-            st.e0 = bp[0];  // last, as on the other side: both sides end with a load into e0
-        }
-    }
-}
-
-// LDS of one K step and of one super-block's scales (one copy: the next super-block's are stored
-// after a barrier that follows the last use of these, which keeps a workgroup under 80 KB of LDS,
-// two of them per CU).
-template <int TN>
-struct KqLds {
-    int8_t A[TM * KP];
-    int8_t B[TN * KP];
+// A step's share of a thread between its global loads and its LDS store (thread t of the K group's NT).
+template <int AP>
+struct KqStage {
+    v4i a[AP];         // activation codes, 16-byte pieces t + NT i: row / 8, part % 8
+    v4i e;             // first half: row t / PR, 8 of its 16 block sums (int16)
+    float dx;          // and its d
+    v4i b[2], q;       // weight columns: 16-byte pieces of low bits (t + NT i: column / 4, part % 4), of high bits (t: column / 2, part % 2)
 };
-template <int TYPE, int TN>
+// The header of a lane's column (Q6_K: its scales and d).
+struct KqHead {
+    v4i h;
+    uint32_t d;
+};
+
+__device__ __forceinline__ uint32_t u32(int x) { return (uint32_t) x; }
+
+// One K group's codes and weight bytes of a step; activation scales of a super-block.
+template <int TYPE, int XT, int WN>
+struct KqCodes {
+    int8_t a[32 * XT * KP];
+    uint8_t b[32 * WN * WP];
+    uint8_t q[TYPE == T_Q4_K ? 16 : 32 * WN * QP];
+};
+template <int TYPE, int XT>
 struct KqScales {
-    int8_t sc[TN][Kq<TYPE>::NSUB];  // Q4_K / Q5_K: the 6-bit sc_j; Q6_K: the 16 int8 scales
-    int8_t mn[Kq<TYPE>::MIN ? TN : 1][8];  // Q4_K / Q5_K: m_j
-    int8_t bh[Kq<TYPE>::MIN ? TM : 1][8], bl[Kq<TYPE>::MIN ? TM : 1][8];  // block sums of sub-block j: 64 bh + bl
-    float dw[TN], dm[Kq<TYPE>::MIN ? TN : 1], dx[TM];
+    float dx[32 * XT];
+    int t128[Kq<TYPE>::BIAS ? 32 * XT : 4];  // 128 times the row's code sum
+    // the block sum of sub-block j as two f16 values: [row][j] its multiple of 64, [row][8 + j] the rest
+    __align__(16) _Float16 bs[Kq<TYPE>::MIN ? 32 * XT : 1][16];
 };
 
-// Byte-wise: codes in [0, 64) minus 32 as int8.
-__device__ __forceinline__ uint32_t minus32(uint32_t v) { return ((v | 0x80808080u) - 0x20202020u) ^ 0x80808080u; }
+template <int TYPE, int XT, int WN, int AP>
+__device__ __forceinline__ void kq_store(const KqStage<AP> & st, KqCodes<TYPE, XT, WN> & L, KqScales<TYPE, XT> & S, int t,
+                                         int h) {
+    constexpr int NT = 64 * WN, PR = NT / (32 * XT);
+#pragma unroll
+    for (int i = 0; i < AP; i++) {
+        const int p = t + NT * i;
+        *reinterpret_cast<v4i *>(L.a + (p >> 3) * KP + 16 * (p & 7)) = st.a[i];
+    }
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+        const int p = t + NT * i;
+        *reinterpret_cast<v4i *>(L.b + (p >> 2) * WP + 16 * (p & 3)) = st.b[i];
+    }
+    if constexpr (TYPE != T_Q4_K) *reinterpret_cast<v4i *>(L.q + (t >> 1) * QP + 16 * (t & 1)) = st.q;
+    if (h != 0) return;
+    const int row = t / PR, part = t % PR;
+    if constexpr (Kq<TYPE>::MIN) {
+        int total = 0;
+        h4_t hi, lo;
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            // bsums 2j and 2j + 1: the two int16 halves of word j
+            const int bs = (int) (int16_t) (st.e[j] & 0xffff) + (st.e[j] >> 16);  // |bs| <= 32 * 128
+            total += bs;
+            hi[j] = (_Float16) (float) (bs & ~63);
+            lo[j] = (_Float16) (float) (bs & 63);
+        }
+        if constexpr (Kq<TYPE>::BIAS) total += __shfl_xor(total, 1, 64);
+        if (part < 2) {
+            *reinterpret_cast<h4_t *>(&S.bs[row][4 * part]) = hi;
+            *reinterpret_cast<h4_t *>(&S.bs[row][8 + 4 * part]) = lo;
+        }
+        if constexpr (Kq<TYPE>::BIAS)
+            if (part == 0) S.t128[row] = 128 * total;
+    }
+    if (part == 0) S.dx[row] = st.dx;
+}
 
-template <int TYPE, int TN>
-__device__ __forceinline__ void kq_store(const KqStage<TYPE> & st, KqLds<TN> & L, KqScales<TYPE, TN> & S, int step) {
-    const int t = threadIdx.x;
-    const int h = step & 1;
-#pragma unroll
-    for (int q = 0; q < 2; q++) {
-        const int c = t + NT * q, row = c >> 3, part = c & 7;
-        *reinterpret_cast<v4i *>(L.A + row * KP + 16 * part) = st.a[q];
-    }
+// Four bytes times a scale below 8 (no carry between bytes: bytes <= 31).
+__device__ __forceinline__ uint32_t bytes_times(uint32_t q, uint32_t s2) {
+    return __builtin_bit_cast(uint32_t, (u16x2) (__builtin_bit_cast(u16x2, q) * __builtin_bit_cast(u16x2, s2)));
+}
+
+// Q6_K: hi and lo codes of four values q (bytes, 0..63) of scale sc.
+__device__ __forceinline__ void q6_hi_lo(uint32_t q, int sc, uint32_t & hi, uint32_t & lo) {
+    const i16x2 s = {(int16_t) sc, (int16_t) sc}, o = s * (int16_t) -32;
+    const i16x2 e = __builtin_bit_cast(i16x2, q & 0x00FF00FFu) * s + o;
+    const i16x2 d = __builtin_bit_cast(i16x2, (q >> 8) & 0x00FF00FFu) * s + o;
+    lo = (__builtin_bit_cast(uint32_t, e) & 0x003F003Fu) | ((__builtin_bit_cast(uint32_t, d) & 0x003F003Fu) << 8);
+    const uint32_t he = __builtin_bit_cast(uint32_t, (i16x2) (e >> 6)), ho = __builtin_bit_cast(uint32_t, (i16x2) (d >> 6));
+    hi = __builtin_amdgcn_perm(ho, he, 0x06020400u);
+}
+
+// The hi and lo operands of piece i of half h for this lane (k half lk of its column): from the low
+// nibbles (o[0], o[1]) and the high ones (o[2], o[3]).
+template <int TYPE>
+__device__ __forceinline__ void kq_expand(const v4i & b, const v4i & q, const KqHead & hd, int h, int i, int lk, v4i (&o)[4]) {
     if constexpr (TYPE == T_Q6_K) {
-        // value r = 32 p + l of the half: low 4 bits from ql (p even: the first 32 bytes, odd: the
-        // second; p < 2 low nibbles, else high), 2 high bits from qh[l] >> 2p
-        if (t < 2 * TN) {
-            const int row = t >> 1, l0 = 16 * (t & 1);
-            v4i o[4];
+        // the low nibbles are values 32 i + 16 lk .. of the half, the high ones those 64 on; their
+        // 16-value sub-blocks 8 h + 2 i + lk and 8 h + 4 + 2 i + lk
+        const int sc0 = (int) (int8_t) (hd.h[2 * h] >> (16 * i + 8 * lk)), sc1 = (int) (int8_t) (hd.h[2 * h + 1] >> (16 * i + 8 * lk));
 #pragma unroll
-            for (int e = 0; e < 4; e++) {
-                const uint32_t x = u32(st.b[e]), y = u32(st.b2[e]), hq = u32(st.b3[e]);
-                o[0][e] = (int) minus32((x & 0x0F0F0F0Fu) | ((hq & 0x03030303u) << 4));
-                o[1][e] = (int) minus32((y & 0x0F0F0F0Fu) | (((hq >> 2) & 0x03030303u) << 4));
-                o[2][e] = (int) minus32(((x >> 4) & 0x0F0F0F0Fu) | (((hq >> 4) & 0x03030303u) << 4));
-                o[3][e] = (int) minus32(((y >> 4) & 0x0F0F0F0Fu) | (((hq >> 6) & 0x03030303u) << 4));
-            }
-#pragma unroll
-            for (int p = 0; p < 4; p++) *reinterpret_cast<v4i *>(L.B + row * KP + 32 * p + l0) = o[p];
+        for (int e = 0; e < 4; e++) {
+            const uint32_t x = u32(b[e]), hq = u32(q[e]) >> (2 * i);
+            uint32_t hi, lo;
+            q6_hi_lo((x & 0x0F0F0F0Fu) | ((hq & 0x03030303u) << 4), sc0, hi, lo);
+            o[0][e] = (int) hi, o[1][e] = (int) lo;
+            q6_hi_lo(((x >> 4) & 0x0F0F0F0Fu) | (hq & 0x30303030u), sc1, hi, lo);
+            o[2][e] = (int) hi, o[3][e] = (int) lo;
         }
-    } else if (t < 4 * TN) {
-        // 16 B of nibbles of chunk c = 2h + u / 2 at bytes l0 = 16 (u % 2): low nibbles are values
-        // 64c + l0 + k, high ones 64c + 32 + l0 + k; Q5_K adds 16 times bit 2c / 2c + 1 of qh[l0 + k]
-        const int row = t >> 2, u = t & 3;
-        const int cc = 2 * h + (u >> 1);
-        v4i lo, hi;
+    } else {
+        // the low nibbles are values 16 lk .. of sub-block 4 h + 2 i, the high ones of the next; 6-bit scales
+        // (get_scale_min_k4): bytes 0..3 of the 12 for j < 4, else byte 4 + j's low nibble and byte j - 4's top bits
+        uint32_t sc0, sc1;
+        const uint32_t q0 = u32(hd.h[1]) >> (16 * i), q2 = u32(hd.h[3]) >> (16 * i);
+        if (h == 0) {
+            sc0 = q0 & 63;
+            sc1 = (q0 >> 8) & 63;
+        } else {
+            sc0 = (q2 & 15) | ((q0 >> 2) & 0x30);
+            sc1 = ((q2 >> 8) & 15) | ((q0 >> 10) & 0x30);
+        }
+        const uint32_t sh0 = (sc0 >> 3) * 0x10001u, sl0 = (sc0 & 7) * 0x10001u;
+        const uint32_t sh1 = (sc1 >> 3) * 0x10001u, sl1 = (sc1 & 7) * 0x10001u;
+        constexpr uint32_t bias = Kq<TYPE>::BIAS ? 0x80808080u : 0u;  // p ^ 0x80 as int8 is p - 128
 #pragma unroll
-        for (int k = 0; k < 4; k++) {
-            const uint32_t x = u32(st.b[k]);
-            uint32_t l = x & 0x0F0F0F0Fu, g = (x >> 4) & 0x0F0F0F0Fu;
+        for (int e = 0; e < 4; e++) {
+            const uint32_t x = u32(b[e]);
+            uint32_t v0 = x & 0x0F0F0F0Fu, v1 = (x >> 4) & 0x0F0F0F0Fu;
             if constexpr (TYPE == T_Q5_K) {
-                const uint32_t hq = u32(st.b2[k]);
-                l |= ((hq >> (2 * cc)) & 0x01010101u) << 4;
-                g |= ((hq >> (2 * cc + 1)) & 0x01010101u) << 4;
+                const uint32_t hq = u32(q[e]) >> (4 * h + 2 * i);
+                v0 |= (hq & 0x01010101u) << 4;
+                v1 |= (hq & 0x02020202u) << 3;
             }
-            lo[k] = (int) l;
-            hi[k] = (int) g;
-        }
-        *reinterpret_cast<v4i *>(L.B + row * KP + 64 * (u >> 1) + 16 * (u & 1)) = lo;
-        *reinterpret_cast<v4i *>(L.B + row * KP + 64 * (u >> 1) + 32 + 16 * (u & 1)) = hi;
-    }
-    if (h == 0) {
-        if (t < TN) {
-            if constexpr (TYPE == T_Q6_K) {
-                *reinterpret_cast<v4i *>(&S.sc[t][0]) = st.e0;
-                S.dw[t] = h2f((uint16_t) st.dw);
-            } else {
-                S.dw[t] = h2f((uint16_t) (u32(st.e0[0]) & 0xffffu));
-                S.dm[t] = h2f((uint16_t) (u32(st.e0[0]) >> 16));
-                const uint32_t q3[3] = {u32(st.e0[1]), u32(st.e0[2]), u32(st.e0[3])};
-#pragma unroll
-                for (int j = 0; j < 8; j++) {
-                    int sc, m;
-                    scale_min(q3, j, sc, m);
-                    S.sc[t][j] = (int8_t) sc;
-                    S.mn[t][j] = (int8_t) m;
-                }
-            }
-        } else if (t < TN + TM) {
-            const int row = t - TN;
-            S.dx[row] = st.dx;
-            if constexpr (Kq<TYPE>::MIN) {
-                const uint32_t bw[8] = {u32(st.e0.x), u32(st.e0.y), u32(st.e0.z), u32(st.e0.w),
-                                        u32(st.e1.x), u32(st.e1.y), u32(st.e1.z), u32(st.e1.w)};
-#pragma unroll
-                for (int j = 0; j < 8; j++) {
-                    // bsums 2j and 2j + 1: the two int16 halves of word j of the 32 bytes
-                    const uint32_t wj = bw[j];
-                    const int bs = (int) (int16_t) (wj & 0xffffu) + (int) (int16_t) (wj >> 16);  // |bs| <= 32 * 127
-                    S.bh[row][j] = (int8_t) (bs >> 6);
-                    S.bl[row][j] = (int8_t) (bs & 63);
-                }
-            }
+            o[0][e] = (int) (bytes_times(v0, sh0) ^ bias);
+            o[1][e] = (int) (bytes_times(v0, sl0) ^ bias);
+            o[2][e] = (int) (bytes_times(v1, sh1) ^ bias);
+            o[3][e] = (int) (bytes_times(v1, sl1) ^ bias);
         }
     }
 }
 
-template <int TYPE, bool RAW, int TN>
-__global__ __launch_bounds__(NT) void k_gemm_kq(const KqArgs<TYPE> a) {
-    constexpr int WN = TN / 32;         // wavefronts along n, each 32 columns
-    constexpr int XT = TM / 32 / (8 / WN);  // 32-row MFMA tiles per wavefront: 2 (TN 128) or 1 (TN 64)
-    __shared__ __align__(16) KqLds<TN> L[2];
-    __shared__ __align__(16) KqScales<TYPE, TN> S;
-    const int mt = (a.M + TM - 1) / TM, nt = (a.N + TN - 1) / TN, total = mt * nt;
-    int id = blockIdx.x;
-    if (total % 8 == 0) id = (id % 8) * (total / 8) + id / 8;  // XCD x holds a contiguous run of tiles
-    const int m0 = (id % mt) * TM, n0 = (id / mt) * TN;
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-    const int wm = wave / WN, wn = wave % WN;  // this wavefront: rows wm * 32 XT + [0, 32 XT), columns wn * 32 + [0, 32)
-    const int lr = lane & 31, lk = lane >> 5;
-    const int nc = wn * 32 + lr;  // the tile column of this lane's outputs
+// 8 unsigned bytes as f16: byte b under the exponent of 1024 is the f16 1024 + b.
+__device__ __forceinline__ h8_t bytes_to_h8(uint32_t b0, uint32_t b1) {
+    h8_t o;
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        const h2_t h = __builtin_bit_cast(h2_t, __builtin_amdgcn_perm(0x64646464u, i < 2 ? b0 : b1, i & 1 ? 0x04030402u : 0x04010400u));
+        o[2 * i] = h.x - (_Float16) 1024.0f;
+        o[2 * i + 1] = h.y - (_Float16) 1024.0f;
+    }
+    return o;
+}
 
-    float acc[XT][16];
-    int i1[XT][16];
+template <int TYPE, int XT, int WN, int KG, bool RAW>
+__global__ __launch_bounds__(64 * WN * KG, 2) void k_gemm_kq(const KqArgs a) {
+    constexpr int TM = 32 * XT, TN = 32 * WN, NT = 64 * WN, AP = 4 * XT / WN;
+    constexpr int SHIFT = TYPE == T_Q6_K ? 6 : 3;
+    constexpr int GM = 8;  // row tiles per group of tiles
+    struct Lds {
+        KqCodes<TYPE, XT, WN> c[2];
+        KqScales<TYPE, XT> s[2];
+    };
+    constexpr size_t kRed = KG > 1 ? (size_t) (KG - 1) * WN * XT * 1024 * 4 : 0;  // the groups' sums
+    constexpr size_t kLds = sizeof(Lds) * KG > kRed ? sizeof(Lds) * KG : kRed;
+    __shared__ __align__(16) uint8_t lds[kLds];
+    const int mt = (a.M + TM - 1) / TM, nt = (a.N + TN - 1) / TN, total = mt * nt;
+    // XCD x holds a contiguous run of tiles; in it, GM row tiles by as many columns as run together, so that
+    // their rows and columns stay in its L2
+    int id = blockIdx.x;
+    if (total % 8 == 0) id = (id % 8) * (total / 8) + id / 8;
+    const int g0 = id / (GM * nt) * GM, gm = min(GM, mt - g0), in = id - g0 * nt;
+    const int m0 = (g0 + in % gm) * TM, n0 = in / gm * TN;
+    const int wave = __builtin_amdgcn_readfirstlane((int) threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const int kg = wave / WN, t = threadIdx.x - kg * NT;
+    const int lr = lane & 31, lk = lane >> 5;
+    const int nw = (wave % WN) * 32, n = n0 + nw + lr;  // this wavefront's columns, this lane's
+    Lds & L = reinterpret_cast<Lds *>(lds)[kg];
+
+    // Where this thread reads. Rows past M or N read the last row (never stored).
+    const int8_t * pa[AP];
+#pragma unroll
+    for (int i = 0; i < AP; i++) {
+        const int p = t + NT * i;
+        pa[i] = a.xc + (size_t) min(m0 + (p >> 3), a.M - 1) * a.nsb * 256 + 16 * (p & 7);
+    }
+    constexpr int PR = NT / TM;
+    const size_t mi = (size_t) min(m0 + t / PR, a.M - 1) * a.nsb;
+    const uint8_t * pb[2];
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+        const int p = t + NT * i;
+        pb[i] = a.w + (size_t) min(n0 + (p >> 2), a.N - 1) * a.nsb * 128 + 16 * (p & 3);
+    }
+    const uint8_t * pq = TYPE == T_Q4_K ? nullptr : a.wqh + (size_t) min(n0 + (t >> 1), a.N - 1) * a.nsb * Kq<TYPE>::QH + 16 * (t & 1);
+    const size_t bi = (size_t) min(n, a.N - 1) * a.nsb;
+    const auto load = [&](KqStage<AP> & s, int sb, int h) {
+#pragma unroll
+        for (int i = 0; i < AP; i++) s.a[i] = *reinterpret_cast<const v4i *>(pa[i] + (size_t) sb * 256 + 128 * h);
+#pragma unroll
+        for (int i = 0; i < 2; i++) s.b[i] = *reinterpret_cast<const v4i *>(pb[i] + (size_t) sb * 128 + 64 * h);
+        if constexpr (TYPE == T_Q5_K) s.q = *reinterpret_cast<const v4i *>(pq + (size_t) sb * 32);
+        if constexpr (TYPE == T_Q6_K) s.q = *reinterpret_cast<const v4i *>(pq + (size_t) sb * 64 + 32 * h);
+        if (h == 0) {
+            s.dx = a.xd[mi + sb];
+            if constexpr (Kq<TYPE>::MIN) s.e = *reinterpret_cast<const v4i *>(a.xbs + (mi + sb) * 16 + 8 * (t & 1));
+        }
+    };
+    const auto load_head = [&](KqHead & hd, int sb) {
+        hd.h = *reinterpret_cast<const v4i *>(a.whdr + (bi + sb) * 16);
+        if constexpr (TYPE == T_Q6_K) hd.d = a.wd[bi + sb];
+    };
+
+    v16f acc[XT];
+    v16i ih[XT], il[XT];
+#pragma unroll
+    for (int x = 0; x < XT; x++) acc[x] = v16f{};
+
+    // This group's super-blocks: the same number of rounds for every group (barriers), a round past the
+    // end computing nothing. Loads past the end read the last super-block again: a load under a
+    // condition makes the compiler wait for every load in flight where the paths meet.
+    const int sb_begin = RAW ? a.raw_sb : min(kg, a.nsb - 1), sb_end = RAW ? a.raw_sb + 1 : a.nsb;
+    const int rounds = RAW ? 1 : (a.nsb + KG - 1) / KG;
+    KqStage<AP> st;
+    KqHead hd, hn;
+    load(st, sb_begin, 0);
+    load_head(hd, sb_begin);
+    kq_store<TYPE, XT, WN>(st, L.c[0], L.s[0], t, 0);
+    load(st, sb_begin, 1);
+    __syncthreads();
+
+    for (int it = 0; it < rounds; it++) {
+        const int sb = RAW ? a.raw_sb : min(kg + it * KG, sb_end - 1), next = min(sb + KG, sb_end - 1), sc = it & 1;
+        const bool on = KG == 1 || kg + it * KG < sb_end;
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            // the next step into the other buffer, the loads of the step after
+            kq_store<TYPE, XT, WN>(st, L.c[h ^ 1], L.s[sc ^ h], t, h ^ 1);
+            load(st, next, h);
+            if (h == 1) load_head(hn, next);
+            if (on) {
+                const KqScales<TYPE, XT> & s = L.s[sc];
+#pragma unroll
+                for (int i = 0; i < 2; i++) {
+                    v4i o[4], q{};
+                    if constexpr (TYPE == T_Q5_K || TYPE == T_Q6_K) q = *reinterpret_cast<const v4i *>(L.c[h].q + (nw + lr) * QP + 16 * lk);
+                    kq_expand<TYPE>(*reinterpret_cast<const v4i *>(L.c[h].b + (nw + lr) * WP + 32 * i + 16 * lk), q, hd, h, i, lk, o);
+#pragma unroll
+                    for (int e = 0; e < 2; e++) {  // low nibbles, high nibbles: 32 values each
+                        const int k0 = TYPE == T_Q6_K ? 32 * i + 64 * e : 64 * i + 32 * e;
+#pragma unroll
+                        for (int x = 0; x < XT; x++) {
+                            const v4i af = *reinterpret_cast<const v4i *>(L.c[h].a + (x * 32 + lr) * KP + k0 + 16 * lk);
+                            const bool first = h == 0 && i == 0 && e == 0;
+                            v16i init{};
+                            if constexpr (Kq<TYPE>::BIAS)
+                                if (first) {
+#pragma unroll
+                                    for (int q = 0; q < 4; q++) {
+                                        const v4i t4 = *reinterpret_cast<const v4i *>(&s.t128[x * 32 + 8 * q + 4 * lk]);
+#pragma unroll
+                                        for (int r = 0; r < 4; r++) init[4 * q + r] = t4[r];
+                                    }
+                                }
+                            ih[x] = __builtin_amdgcn_mfma_i32_32x32x32_i8(af, o[2 * e], first ? init : ih[x], 0, 0, 0);
+                            il[x] = __builtin_amdgcn_mfma_i32_32x32x32_i8(af, o[2 * e + 1], first ? init : il[x], 0, 0, 0);
+                        }
+                    }
+                }
+                if (h == 1) {  // the super-block is complete: its integer parts into the f32 sums
+                    h8_t bm{};
+                    float dw, dm = 0.0f;
+                    if constexpr (Kq<TYPE>::MIN) {
+                        dw = h2f((uint16_t) (u32(hd.h[0]) & 0xffffu));
+                        dm = h2f((uint16_t) (u32(hd.h[0]) >> 16));
+                        asm volatile("" : "+v"(dm));  // an f32 register: from f16 the multiply-adds take the mixed form, half the rate
+                        // mins: bytes 4..7 (6 bits) of the 12; then byte 8 + j's high nibble with byte 4 + j's top two bits
+                        const uint32_t q1 = u32(hd.h[2]), q2 = u32(hd.h[3]);
+                        bm = bytes_to_h8(q1 & 0x3F3F3F3Fu, ((q2 >> 4) & 0x0F0F0F0Fu) | ((q1 >> 2) & 0x30303030u));
+                    } else {
+                        dw = h2f((uint16_t) hd.d);
+                    }
+#pragma unroll
+                    for (int x = 0; x < XT; x++) {
+                        // I2 = sum_j m_j(n) bs_j(m): lanes 0..31 the multiples of 64, lanes 32..63 the rest
+                        v16f i2{};
+                        if constexpr (Kq<TYPE>::MIN) {
+                            const h8_t as = *reinterpret_cast<const h8_t *>(&s.bs[x * 32 + lr][8 * lk]);
+                            i2 = __builtin_amdgcn_mfma_f32_32x32x16_f16(as, bm, v16f{}, 0, 0, 0);
+                        }
+                        if constexpr (RAW) {  // the one super-block's integers, stored here
+#pragma unroll
+                            for (int r = 0; r < 16; r++) {
+                                const int m = m0 + x * 32 + 8 * (r >> 2) + 4 * lk + (r & 3);
+                                if (m >= a.M || n >= a.N) continue;
+                                int32_t * out = a.raw + ((size_t) m * a.N + n) * (Kq<TYPE>::MIN ? 2 : 1);
+                                out[0] = (ih[x][r] << SHIFT) + il[x][r];
+                                if constexpr (Kq<TYPE>::MIN) out[1] = (int) i2[r];
+                            }
+                        } else {
+#pragma unroll
+                            for (int q = 0; q < 4; q++) {
+                                // d_x of this lane's rows: element 4 q + r is row 8 q + 4 lk + r of the MFMA tile
+                                const float4 d4 = *reinterpret_cast<const float4 *>(&s.dx[x * 32 + 8 * q + 4 * lk]);
+                                const float dx[4] = {d4.x, d4.y, d4.z, d4.w};
+#pragma unroll
+                                for (int r = 0; r < 4; r++) {
+                                    const int e = 4 * q + r;
+                                    float v = dw * (float) ((ih[x][e] << SHIFT) + il[x][e]);
+                                    if constexpr (Kq<TYPE>::MIN) v = fmaf(-dm, i2[e], v);
+                                    acc[x][e] = fmaf(dx[r], v, acc[x][e]);
+                                }
+                            }
+                        }
+                    }
+                }
+            }
+            if (h == 1) hd = hn;
+            __syncthreads();
+        }
+    }
+    if constexpr (RAW) return;
+
+    if constexpr (KG > 1) {  // groups 1.. hand their sums to group 0, added in the groups' order
+        float * red = reinterpret_cast<float *>(lds) + (size_t) (wave % WN) * XT * 1024 + lane;
+        if (kg > 0) {
+#pragma unroll
+            for (int x = 0; x < XT; x++)
+#pragma unroll
+                for (int r = 0; r < 16; r++) red[(size_t) (kg - 1) * WN * XT * 1024 + x * 1024 + r * 64] = acc[x][r];
+        }
+        __syncthreads();
+        if (kg > 0) return;
+        for (int g = 0; g < KG - 1; g++)
+#pragma unroll
+            for (int x = 0; x < XT; x++)
+#pragma unroll
+                for (int r = 0; r < 16; r++) acc[x][r] += red[(size_t) g * WN * XT * 1024 + x * 1024 + r * 64];
+    }
+    if (n >= a.N) return;
 #pragma unroll
     for (int x = 0; x < XT; x++)
 #pragma unroll
-        for (int r = 0; r < 16; r++) acc[x][r] = 0.0f, i1[x][r] = 0;
-
-    const int s_begin = RAW ? 2 * a.raw_sb : 0, s_end = RAW ? 2 * a.raw_sb + 2 : 2 * a.nsb;
-    KqStage<TYPE> st;
-    kq_load<TYPE, TN>(st, a, m0, n0, s_begin);
-    kq_store<TYPE, TN>(st, L[0], S, s_begin);
-    __syncthreads();
-
-    for (int step = s_begin; step < s_end; step++) {
-        const int buf = (step - s_begin) & 1, h = step & 1;
-        if (step + 1 < s_end) kq_load<TYPE, TN>(st, a, m0, n0, step + 1);
-        const KqLds<TN> & l = L[buf];
-        if constexpr (TYPE == T_Q6_K) {
-#pragma unroll
-            for (int jj = 0; jj < 8; jj++) {  // sub-blocks of 16: v_mfma_i32_32x32x16_i8
-                long af[XT];
-#pragma unroll
-                for (int x = 0; x < XT; x++)
-                    af[x] = *reinterpret_cast<const long *>(l.A + (wm * 32 * XT + x * 32 + lr) * KP + 16 * jj + 8 * lk);
-                const long bf = *reinterpret_cast<const long *>(l.B + nc * KP + 16 * jj + 8 * lk);
-                const int sc = S.sc[nc][8 * h + jj];
-#pragma unroll
-                for (int x = 0; x < XT; x++) {
-                    const v16i c = __builtin_amdgcn_mfma_i32_32x32x16_i8(af[x], bf, v16i{}, 0, 0, 0);
-#pragma unroll
-                    for (int r = 0; r < 16; r++) i1[x][r] += sc * c[r];
-                }
-            }
-        } else {
-#pragma unroll
-            for (int jj = 0; jj < 4; jj++) {  // sub-blocks of 32: v_mfma_i32_32x32x32_i8
-                v4i af[XT];
-#pragma unroll
-                for (int x = 0; x < XT; x++)
-                    af[x] = *reinterpret_cast<const v4i *>(l.A + (wm * 32 * XT + x * 32 + lr) * KP + 32 * jj + 16 * lk);
-                const v4i bf = *reinterpret_cast<const v4i *>(l.B + nc * KP + 32 * jj + 16 * lk);
-                const int sc = S.sc[nc][4 * h + jj];
-#pragma unroll
-                for (int x = 0; x < XT; x++) {
-                    const v16i c = __builtin_amdgcn_mfma_i32_32x32x32_i8(af[x], bf, v16i{}, 0, 0, 0);
-#pragma unroll
-                    for (int r = 0; r < 16; r++) i1[x][r] += sc * c[r];
-                }
-            }
+        for (int r = 0; r < 16; r++) {
+            const int m = m0 + x * 32 + 8 * (r >> 2) + 4 * lk + (r & 3);
+            if (m >= a.M) continue;
+            const size_t o = (size_t) m * a.ldy + n;
+            a.y[o] = a.res ? acc[x][r] + a.res[o] : acc[x][r];
         }
-        if (h == 1) {  // the super-block is complete: its integer parts into the f32 sums
-            v16i i2[XT];
-            if constexpr (Kq<TYPE>::MIN) {
-                // I2 = sum_j m_j(n) bs_j(m) = 64 (bh . mn) + (bl . mn), K = 8 of 32 (lanes 32..63 and
-                // bytes 8..15 zero)
-                const int keep = lk ? 0 : -1;
-                const int2 m8 = *reinterpret_cast<const int2 *>(&S.mn[nc][0]);
-                const v4i bm = v4i{m8.x & keep, m8.y & keep, 0, 0};
-#pragma unroll
-                for (int x = 0; x < XT; x++) {
-                    const int row = wm * 32 * XT + x * 32 + lr;
-                    const int2 h8 = *reinterpret_cast<const int2 *>(&S.bh[row][0]);
-                    const int2 l8 = *reinterpret_cast<const int2 *>(&S.bl[row][0]);
-                    const v4i ah = v4i{h8.x & keep, h8.y & keep, 0, 0};
-                    const v4i al = v4i{l8.x & keep, l8.y & keep, 0, 0};
-                    const v16i hh = __builtin_amdgcn_mfma_i32_32x32x32_i8(ah, bm, v16i{}, 0, 0, 0);
-                    const v16i ll = __builtin_amdgcn_mfma_i32_32x32x32_i8(al, bm, v16i{}, 0, 0, 0);
-#pragma unroll
-                    for (int r = 0; r < 16; r++) i2[x][r] = 64 * hh[r] + ll[r];
-                }
-            }
-            if constexpr (RAW) {  // the one super-block's integers, stored here
-                const int n = n0 + nc;
-#pragma unroll
-                for (int x = 0; x < XT; x++)
-#pragma unroll
-                    for (int r = 0; r < 16; r++) {
-                        const int m = m0 + wm * 32 * XT + x * 32 + 8 * (r >> 2) + 4 * lk + (r & 3);
-                        if (m >= a.M || n >= a.N) continue;
-                        int32_t * o = a.raw + ((size_t) m * a.N + n) * (Kq<TYPE>::MIN ? 2 : 1);
-                        o[0] = i1[x][r];
-                        if constexpr (Kq<TYPE>::MIN) o[1] = i2[x][r];
-                    }
-            } else {
-                const float dw = S.dw[nc], dm = Kq<TYPE>::MIN ? S.dm[nc] : 0.0f;
-#pragma unroll
-                for (int x = 0; x < XT; x++) {
-                    // d_x of this lane's rows: element r is row wm*64 + x*32 + 8 (r / 4) + 4 lk + r % 4
-                    float4 dxv[4];
-#pragma unroll
-                    for (int q = 0; q < 4; q++)
-                        dxv[q] = *reinterpret_cast<const float4 *>(&S.dx[wm * 32 * XT + x * 32 + 8 * q + 4 * lk]);
-#pragma unroll
-                    for (int r = 0; r < 16; r++) {
-                        const float4 d4 = dxv[r >> 2];
-                        const float dx = (r & 3) == 0 ? d4.x : (r & 3) == 1 ? d4.y : (r & 3) == 2 ? d4.z : d4.w;
-                        float v = dw * (float) i1[x][r];
-                        if constexpr (Kq<TYPE>::MIN) v = fmaf(-dm, (float) i2[x][r], v);
-                        acc[x][r] = fmaf(dx, v, acc[x][r]);
-                        i1[x][r] = 0;
-                    }
-                }
-            }
-        }
-        if (step + 1 < s_end) {
-            if (h == 1) __syncthreads();  // every wavefront is done with this super-block's scales
-            kq_store<TYPE, TN>(st, L[buf ^ 1], S, step + 1);
-        }
-        __syncthreads();
-    }
-
-    if constexpr (!RAW) {
-        const int n = n0 + nc;
-        if (n >= a.N) return;
-#pragma unroll
-        for (int x = 0; x < XT; x++) {
-#pragma unroll
-            for (int r = 0; r < 16; r++) {
-                const int m = m0 + wm * 32 * XT + x * 32 + 8 * (r >> 2) + 4 * lk + (r & 3);
-                if (m >= a.M) continue;
-                const size_t o = (size_t) m * a.ldy + n;
-                a.y[o] = a.res ? acc[x][r] + a.res[o] : acc[x][r];
-            }
-        }
-    }
 }
 
 template <int TYPE, bool RAW>
 void run_kq(const void * wv, int64_t N, int64_t K, const void * act, int64_t M, float * y, int64_t ldy,
             const float * res, int32_t * raw, int raw_sb, hipStream_t s) {
-    // 64-column tiles when 128-column ones would leave CUs without a workgroup
-    const bool narrow = ((M + TM - 1) / TM) * ((N + 127) / 128) <= cu_count();
-    const int TN = narrow ? 64 : 128;
     const WeightLayout WL = weight_layout(TYPE, N, K);
     const ActLayout AL = act_layout(TYPE, M, K);
     const uint8_t * w = (const uint8_t *) wv;
     const uint8_t * x = (const uint8_t *) act;
-    KqArgs<TYPE> a{};
+    KqArgs a{};
     a.w = w + WL.qs;
     a.wd = TYPE == T_Q6_K ? (const uint16_t *) (w + WL.d) : nullptr;
     a.wqh = TYPE == T_Q4_K ? nullptr : w + WL.qh;
@@ -404,9 +440,18 @@ void run_kq(const void * wv, int64_t N, int64_t K, const void * act, int64_t M, 
     a.nsb = (int) (K / 256);
     a.ldy = (int) ldy;
     a.raw_sb = raw_sb;
-    const unsigned grid = (unsigned) (((M + TM - 1) / TM) * ((N + TN - 1) / TN));
-    if (narrow) k_gemm_kq<TYPE, RAW, 64><<<grid, NT, 0, s>>>(a);
-    else k_gemm_kq<TYPE, RAW, 128><<<grid, NT, 0, s>>>(a);
+    const auto tiles = [&](int64_t tm, int64_t tn) { return ((M + tm - 1) / tm) * ((N + tn - 1) / tn); };
+    // 64 x 128 tiles when there are more of them than CUs; else 64 x 64 in two K groups; when even those
+    // cover less than half the CUs, 32 x 32 in eight (512 x 4096 x 14336: 94 us in 512 tiles of 64 x 64,
+    // 114 in 256 of 64 x 128 without groups; 128 x 4096 x 4096: 17 us in 512 tiles of 32 x 32, 24 in 128
+    // of 64 x 64 without groups)
+    if constexpr (RAW) {
+        k_gemm_kq<TYPE, 2, 4, 1, RAW><<<(unsigned) tiles(64, 128), 256, 0, s>>>(a);
+    } else {
+        if (tiles(64, 128) > cu_count()) k_gemm_kq<TYPE, 2, 4, 1, RAW><<<(unsigned) tiles(64, 128), 256, 0, s>>>(a);
+        else if (tiles(64, 64) > cu_count() / 2) k_gemm_kq<TYPE, 2, 2, 2, RAW><<<(unsigned) tiles(64, 64), 256, 0, s>>>(a);
+        else k_gemm_kq<TYPE, 1, 1, 8, RAW><<<(unsigned) tiles(32, 32), 512, 0, s>>>(a);
+    }
 }
 
 }  // namespace
