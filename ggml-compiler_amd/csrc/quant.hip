@@ -2,9 +2,9 @@
 //
 // Weight encoders produce ggml's block bytes exactly (the ggml_compiler_quantize contract,
 // runtime/include/ggml_compiler_rt.h:83-87, whose CPU implementation is ggml_quantize_chunk with
-// no importance matrix, runtime/src/ggml_compiler_rt.cpp:859-876). They run one thread per block
-// (one per 256-super-block for the K-quants) in ggml's sequential order with contraction off, so every
-// float operation rounds as the C reference does. Activation quantizers produce the vec_dot_type
+// no importance matrix, runtime/src/ggml_compiler_rt.cpp:859-876). They run eight lanes per block
+// (Q8_0, Q4_0) or one per sub-block (the K-quants), every float sum in ggml's sequential order with
+// contraction off, so every float operation rounds as the C reference does. Activation quantizers produce the vec_dot_type
 // that ggml-cpu converts src1 into before a quantized mul_mat (Q8_0 for Q4_0/Q8_0 weights, Q8_K
 // for Q4_K / Q5_K / Q6_K), in the device "act" layout described in gcq_common.h.
 #include "gcq_common.h"
@@ -13,64 +13,107 @@ namespace gcq {
 
 // ----------------------------------------------------------------------- weight encoders
 
-// ggml quantize_row_q8_0_ref: d = amax/127, q = roundf(x * (1/d)).
+// Stores to ggml's block bytes, whose blocks (18, 34, 210 bytes) and caller's buffer keep no
+// alignment: one unaligned store of the whole piece.
+template <class T>
+__device__ __forceinline__ void put(uint8_t * o, T v) { __builtin_memcpy(o, &v, sizeof v); }
+__device__ __forceinline__ float4 get4(const float * x) {
+    float4 v;
+    __builtin_memcpy(&v, x, sizeof v);
+    return v;
+}
+
+// ggml quantize_row_q8_0_ref: d = amax/127, q = roundf(x * (1/d)). Eight lanes per block, 4 values each
+// (a thread per block had its loads 128 bytes apart and 34 byte stores: 4096 x 14336 101 us, so 57).
 __global__ void k_enc_q8_0(const float * __restrict__ x, uint8_t * __restrict__ out, int64_t nblocks) {
 #pragma clang fp contract(off)
-    const int64_t i = (int64_t) blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= nblocks) return;
-    const float * xb = x + i * QK;
+    const int64_t t = (int64_t) blockIdx.x * blockDim.x + threadIdx.x, i = t >> 3;
+    if (i >= nblocks) return;  // whole 8-lane groups
+    const int s = (int) (t & 7);
+    const float4 v4 = get4(x + t * 4);
+    const float v[4] = {v4.x, v4.y, v4.z, v4.w};
     float amax = 0.0f;
-    for (int j = 0; j < QK; j++) amax = fmaxf(amax, fabsf(xb[j]));
+    for (int j = 0; j < 4; j++) amax = fmaxf(amax, fabsf(v[j]));
+    for (int o = 1; o < 8; o <<= 1) amax = fmaxf(amax, __shfl_xor(amax, o, 64));
     const float d = __fdiv_rn(amax, 127.0f);
     const float id = d != 0.0f ? __fdiv_rn(1.0f, d) : 0.0f;
     uint8_t * o = out + i * 34;
-    const uint16_t dh = f2h_exact(d);
-    o[0] = (uint8_t) dh;
-    o[1] = (uint8_t) (dh >> 8);
-    for (int j = 0; j < QK; j++) o[2 + j] = (uint8_t) (int8_t) roundf(xb[j] * id);
+    if (s == 0) put(o, f2h_exact(d));
+    uint32_t w = 0;
+    for (int j = 0; j < 4; j++) w |= (uint32_t) (uint8_t) (int8_t) roundf(v[j] * id) << (8 * j);
+    put(o + 2 + 4 * s, w);
 }
 
 // ggml quantize_row_q4_0_ref: d = (first largest-|x| value)/-8, q = min(15, trunc(x/d + 8.5)).
+// Eight lanes per block, 4 values each; byte j holds the codes of values j and j + 16.
 __global__ void k_enc_q4_0(const float * __restrict__ x, uint8_t * __restrict__ out, int64_t nblocks) {
 #pragma clang fp contract(off)
-    const int64_t i = (int64_t) blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= nblocks) return;
-    const float * xb = x + i * QK;
+    const int64_t t = (int64_t) blockIdx.x * blockDim.x + threadIdx.x, i = t >> 3;
+    if (i >= nblocks) return;  // whole 8-lane groups
+    const int s = (int) (t & 7);
+    const float4 v4 = get4(x + t * 4);
+    const float v[4] = {v4.x, v4.y, v4.z, v4.w};
     float amax = 0.0f, max = 0.0f;
-    for (int j = 0; j < QK; j++) {
-        const float a = fabsf(xb[j]);
+    int at = 32;
+    for (int j = 0; j < 4; j++) {
+        const float a = fabsf(v[j]);
         if (amax < a) {
             amax = a;
-            max = xb[j];
+            max = v[j];
+            at = 4 * s + j;
+        }
+    }
+    for (int o = 1; o < 8; o <<= 1) {  // the largest |x|, ties to the lowest index
+        const float a2 = __shfl_xor(amax, o, 64), m2 = __shfl_xor(max, o, 64);
+        const int at2 = __shfl_xor(at, o, 64);
+        if (amax < a2 || (amax == a2 && at2 < at)) {
+            amax = a2;
+            max = m2;
+            at = at2;
         }
     }
     const float d = __fdiv_rn(max, -8.0f);
     const float id = d != 0.0f ? __fdiv_rn(1.0f, d) : 0.0f;
     uint8_t * o = out + i * 18;
-    const uint16_t dh = f2h_exact(d);
-    o[0] = (uint8_t) dh;
-    o[1] = (uint8_t) (dh >> 8);
-    for (int j = 0; j < QK / 2; j++) {
-        int lo = (int) (xb[j] * id + 8.5f);
-        int hi = (int) (xb[j + 16] * id + 8.5f);
-        lo = lo < 15 ? lo : 15;
-        hi = hi < 15 ? hi : 15;
-        o[2 + j] = (uint8_t) (lo | (hi << 4));
+    if (s == 0) put(o, f2h_exact(d));
+    uint32_t w = 0;
+    for (int j = 0; j < 4; j++) {
+        int q = (int) (v[j] * id + 8.5f);
+        q = q < 15 ? q : 15;
+        w |= (uint32_t) (uint8_t) (q << (s < 4 ? 0 : 4)) << (8 * j);
     }
+    w |= __shfl_xor(w, 4, 64);
+    if (s < 4) put(o + 2 + 4 * s, w);
 }
 
 __device__ __forceinline__ int near_int(float v) { return __float2int_rn(v); }
 
+// The code of v as ggml's near_int then a clamp gives it, as a float (a NaN's is 0, as its conversion to int).
+template <int LO, int HI>
+__device__ __forceinline__ float code(float v) {
+    if (LO < 0) v = v == v ? v : 0.0f;
+    return fminf(fmaxf(__builtin_rintf(v), (float) LO), (float) HI);
+}
+
+// The K-quant encoders run a thread per sub-block, its 32 (16) values, weights and codes in
+// registers, every sum in the reference's order; the 8 (16) lanes of a super-block then exchange
+// scales and codes. What bounds them is the VALU: 21 candidates of 32 values, 17 operations each
+// (Q4_K). 4096 x 14336 values: Q4_K 5716 -> 530 us, Q5_K 4763 -> 410, Q6_K 482 -> 280 against a thread per
+// super-block with its arrays in scratch memory. The 146 registers leave three wavefronts per SIMD;
+// held to 128 for a fourth it spills: 590-720 us.
+
 // ggml make_qkx2_quants(32, NMAX, x, w, L, &min, Laux, rmin, 0.1, NSTEP, false): weighted
 // least-squares (scale, min) over NSTEP + 1 candidate inverse scales. Sequential, as the C
-// reference. Q4_K: NMAX 15, rmin -1, NSTEP 20; Q5_K: NMAX 31, rmin -0.5, NSTEP 15.
+// reference. Q4_K: NMAX 15, rmin -1, NSTEP 20; Q5_K: NMAX 31, rmin -0.5, NSTEP 15. The codes are
+// those of the inverse scale l_iscale from l_min (l_iscale 0: all zero).
 template <int NMAX, int NSTEP>
-__device__ float qkx2_fit(const float * x, const float * w, uint8_t * L, float * the_min, float rmin) {
+__device__ __forceinline__ float qkx2_fit(const float (&x)[32], const float (&w)[32], float & l_iscale, float & l_min,
+                                          float & the_min, float rmin) {
 #pragma clang fp contract(off)
-    uint8_t Laux[32];
     float min = x[0], max = x[0];
     float sum_w = w[0];
     float sum_x = sum_w * x[0];
+#pragma unroll
     for (int i = 1; i < 32; i++) {
         if (x[i] < min) min = x[i];
         if (x[i] > max) max = x[i];
@@ -79,33 +122,36 @@ __device__ float qkx2_fit(const float * x, const float * w, uint8_t * L, float *
         sum_x += wi * x[i];
     }
     if (min > 0) min = 0;
+    l_min = min;
     if (max == min) {
-        for (int i = 0; i < 32; i++) L[i] = 0;
-        *the_min = -min;
+        l_iscale = 0.0f;
+        the_min = -min;
         return 0.0f;
     }
-    float iscale = __fdiv_rn((float) NMAX, max - min);
+    const float range = max - min;
+    float min_now = min;
+    float iscale = __fdiv_rn((float) NMAX, range);
     float scale = __fdiv_rn(1.0f, iscale);
     float best = 0;
+    l_iscale = iscale;
+#pragma unroll
     for (int i = 0; i < 32; i++) {
-        int l = near_int(iscale * (x[i] - min));
-        l = l < 0 ? 0 : (l > NMAX ? NMAX : l);
-        L[i] = (uint8_t) l;
-        const float diff = scale * (float) L[i] + min - x[i];
+        const float l = code<0, NMAX>(iscale * (x[i] - min));
+        const float diff = scale * l + min - x[i];
         best += w[i] * (diff * diff);
     }
     for (int is = 0; is <= NSTEP; is++) {
-        iscale = __fdiv_rn(rmin + 0.1f * (float) is + (float) NMAX, max - min);
+        // the reference divides by max - min with the min as the fits have moved it
+        iscale = __fdiv_rn(rmin + 0.1f * (float) is + (float) NMAX, max - min_now);
+        float l[32];
         float sum_l = 0, sum_l2 = 0, sum_xl = 0;
+#pragma unroll
         for (int i = 0; i < 32; i++) {
-            int l = near_int(iscale * (x[i] - min));
-            l = l < 0 ? 0 : (l > NMAX ? NMAX : l);
-            Laux[i] = (uint8_t) l;
-            const float wi = w[i];
-            const float lf = (float) l;
-            sum_l += wi * lf;
-            sum_l2 += wi * lf * lf;
-            sum_xl += wi * lf * x[i];
+            l[i] = code<0, NMAX>(iscale * (x[i] - min_now));
+            const float wl = w[i] * l[i];
+            sum_l += wl;
+            sum_l2 += wl * l[i];
+            sum_xl += wl * x[i];
         }
         const float D = sum_w * sum_l2 - sum_l * sum_l;
         if (D > 0) {
@@ -116,19 +162,21 @@ __device__ float qkx2_fit(const float * x, const float * w, uint8_t * L, float *
                 this_scale = __fdiv_rn(sum_xl, sum_l2);
             }
             float mad = 0;
+#pragma unroll
             for (int i = 0; i < 32; i++) {
-                const float diff = this_scale * (float) Laux[i] + this_min - x[i];
+                const float diff = this_scale * l[i] + this_min - x[i];
                 mad += w[i] * (diff * diff);
             }
             if (mad < best) {
-                for (int i = 0; i < 32; i++) L[i] = Laux[i];
+                l_iscale = iscale;
+                l_min = min_now;
                 best = mad;
                 scale = this_scale;
-                min = this_min;
+                min_now = this_min;
             }
         }
     }
-    *the_min = -min;
+    the_min = -min_now;
     return scale;
 }
 
@@ -142,140 +190,115 @@ __device__ __forceinline__ void scale_min_k4(int j, const uint8_t * q, int & sc,
     }
 }
 
-// The 6-bit (scale, min) pairs of a Q4_K / Q5_K super-block, relative to its largest scale and
-// min (ggml quantize_row_q4_K_ref / q5_K_ref): writes scales[12], returns fp16 (d, dmin).
-__device__ void pack_scale_min_k4(const float * scales, const float * mins, float max_scale, float max_min,
-                                  uint8_t * sb, uint16_t & dh, uint16_t & mh) {
+// ggml quantize_row_q4_K_ref / quantize_row_q5_K_ref, eight lanes per 256-value super-block, a 32-value
+// sub-block each: the sub-block fits; the 6-bit (scale, min) pairs relative to the super-block's
+// largest (scales[12], fp16 d and dmin); codes recomputed against the rounded scales. Q5_K: 5-bit
+// codes, the fifth bit of value l of sub-block j in bit j of qh[l].
+template <int TYPE>
+__global__ __launch_bounds__(256) void k_enc_kq(const float * __restrict__ xall, uint8_t * __restrict__ out,
+                                                int64_t nblocks) {
 #pragma clang fp contract(off)
+    constexpr int NMAX = TYPE == T_Q4_K ? 15 : 31;
+    const int64_t t = (int64_t) blockIdx.x * blockDim.x + threadIdx.x, i = t >> 3;
+    if (i >= nblocks) return;  // whole 8-lane groups
+    const int j = (int) (t & 7), lane0 = (threadIdx.x & 63) & ~7;
+    float x[32], w[32];
+#pragma unroll
+    for (int q = 0; q < 8; q++) {
+        const float4 v = get4(xall + t * 32 + 4 * q);
+        x[4 * q] = v.x, x[4 * q + 1] = v.y, x[4 * q + 2] = v.z, x[4 * q + 3] = v.w;
+    }
+    float sum_x2 = 0;
+#pragma unroll
+    for (int l = 0; l < 32; l++) sum_x2 += x[l] * x[l];
+    const float av_x = sqrtf(__fdiv_rn(sum_x2, 32.0f));  // IEEE sqrt: __fsqrt_rn is the native approximation here
+#pragma unroll
+    for (int l = 0; l < 32; l++) w[l] = av_x + fabsf(x[l]);
+    float l_iscale, l_min, min;
+    const float scale = TYPE == T_Q4_K ? qkx2_fit<15, 20>(x, w, l_iscale, l_min, min, -1.0f)
+                                       : qkx2_fit<31, 15>(x, w, l_iscale, l_min, min, -0.5f);
+    float max_scale = scale > 0 ? scale : 0.0f, max_min = min > 0 ? min : 0.0f;
+    for (int o = 1; o < 8; o <<= 1) {
+        max_scale = fmaxf(max_scale, __shfl_xor(max_scale, o, 64));
+        max_min = fmaxf(max_min, __shfl_xor(max_min, o, 64));
+    }
     const float inv_scale = max_scale > 0 ? __fdiv_rn(63.f, max_scale) : 0.f;
     const float inv_min = max_min > 0 ? __fdiv_rn(63.f, max_min) : 0.f;
-    for (int j = 0; j < 12; j++) sb[j] = 0;
-    for (int j = 0; j < 8; j++) {
-        int ls = near_int(inv_scale * scales[j]);
-        int lm = near_int(inv_min * mins[j]);
-        ls = ls > 63 ? 63 : ls;
-        lm = lm > 63 ? 63 : lm;
-        if (j < 4) {
-            sb[j] = (uint8_t) ls;
-            sb[j + 4] = (uint8_t) lm;
-        } else {
-            sb[j + 4] = (uint8_t) ((ls & 0xF) | ((lm & 0xF) << 4));
-            sb[j - 4] |= (uint8_t) ((ls >> 4) << 6);
-            sb[j] |= (uint8_t) ((lm >> 4) << 6);
-        }
-    }
-    dh = f2h_exact(__fdiv_rn(max_scale, 63.f));
-    mh = f2h_exact(__fdiv_rn(max_min, 63.f));
-}
-
-// ggml quantize_row_q4_K_ref, one thread per 256-value super-block.
-__global__ void k_enc_q4_K(const float * __restrict__ xall, uint8_t * __restrict__ out, int64_t nblocks) {
-#pragma clang fp contract(off)
-    const int64_t i = (int64_t) blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= nblocks) return;
-    const float * x = xall + i * QKK;
-    uint8_t L[QKK];
-    float w[32], mins[8], scales[8];
-    float max_scale = 0, max_min = 0;
-    for (int j = 0; j < 8; j++) {
-        float sum_x2 = 0;
-        for (int l = 0; l < 32; l++) sum_x2 += x[32 * j + l] * x[32 * j + l];
-        const float av_x = sqrtf(__fdiv_rn(sum_x2, 32.0f));  // IEEE sqrt: __fsqrt_rn is the native approximation here
-        for (int l = 0; l < 32; l++) w[l] = av_x + fabsf(x[32 * j + l]);
-        scales[j] = qkx2_fit<15, 20>(x + 32 * j, w, L + 32 * j, &mins[j], -1.0f);
-        if (scales[j] > max_scale) max_scale = scales[j];
-        if (mins[j] > max_min) max_min = mins[j];
-    }
+    // as bytes, then 6 bits: the packing keeps no more of a scale than its low 8 bits
+    int ls = near_int(inv_scale * scale), lm = near_int(inv_min * min);
+    ls = ls > 63 ? 63 : ls;
+    lm = lm > 63 ? 63 : lm;
+    const uint16_t dh = f2h_exact(__fdiv_rn(max_scale, 63.f)), mh = f2h_exact(__fdiv_rn(max_min, 63.f));
     uint8_t sb[12];
-    uint16_t dh, mh;
-    pack_scale_min_k4(scales, mins, max_scale, max_min, sb, dh, mh);
-    for (int j = 0; j < 8; j++) {
-        int sc, m;
-        scale_min_k4(j, sb, sc, m);
-        const float d = h2f(dh) * (float) sc;
-        if (d == 0.0f) continue;  // the fit's codes stay, as in ggml
-        const float dm = h2f(mh) * (float) m;
-        for (int l = 0; l < 32; l++) {
-            int q = near_int(__fdiv_rn(x[32 * j + l] + dm, d));
-            L[32 * j + l] = (uint8_t) (q < 0 ? 0 : (q > 15 ? 15 : q));
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        const int s0 = __shfl(ls, lane0 + k, 64), m0 = __shfl(lm, lane0 + k, 64);
+        const int s1 = __shfl(ls, lane0 + 4 + k, 64), m1 = __shfl(lm, lane0 + 4 + k, 64);
+        sb[k] = (uint8_t) ((uint8_t) s0 | (uint8_t) ((s1 >> 4) << 6));
+        sb[4 + k] = (uint8_t) ((uint8_t) m0 | (uint8_t) ((m1 >> 4) << 6));
+        sb[8 + k] = (uint8_t) ((s1 & 0xF) | ((m1 & 0xF) << 4));
+    }
+    int sc = 0, m = 0;
+#pragma unroll
+    for (int k = 0; k < 8; k++) {
+        int sk, mk;
+        scale_min_k4(k, sb, sk, mk);
+        sc = k == j ? sk : sc;
+        m = k == j ? mk : m;
+    }
+    const float d = h2f(dh) * (float) sc, dm = h2f(mh) * (float) m;
+    uint32_t c[8];  // codes, 4 to a word
+#pragma unroll
+    for (int q = 0; q < 8; q++) {
+        c[q] = 0;
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            const float v = x[4 * q + e];
+            // d == 0: the fit's codes stay, as in ggml
+            const float l = d == 0.0f ? (l_iscale == 0.0f ? 0.0f : code<0, NMAX>(l_iscale * (v - l_min)))
+                                      : code<0, NMAX>(__fdiv_rn(v + dm, d));
+            c[q] |= (uint32_t) (int) l << (8 * e);
         }
     }
-    uint8_t * o = out + i * 144;
-    o[0] = (uint8_t) dh;
-    o[1] = (uint8_t) (dh >> 8);
-    o[2] = (uint8_t) mh;
-    o[3] = (uint8_t) (mh >> 8);
-    for (int j = 0; j < 12; j++) o[4 + j] = sb[j];
-    for (int c = 0; c < 4; c++)
-        for (int l = 0; l < 32; l++) o[16 + 32 * c + l] = (uint8_t) (L[64 * c + l] | (L[64 * c + 32 + l] << 4));
-}
-
-// ggml quantize_row_q5_K_ref, one thread per 256-value super-block: the Q4_K fit with 5-bit codes
-// (make_qkx2_quants(32, 31, ..., -0.5, 0.1, 15)), the fifth bit of value 64c + l (c < 4, l < 64)
-// in bit 2c + (l >= 32) of qh[l % 32].
-__global__ void k_enc_q5_K(const float * __restrict__ xall, uint8_t * __restrict__ out, int64_t nblocks) {
-#pragma clang fp contract(off)
-    const int64_t i = (int64_t) blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= nblocks) return;
-    const float * x = xall + i * QKK;
-    uint8_t L[QKK];
-    float w[32], mins[8], scales[8];
-    float max_scale = 0, max_min = 0;
-    for (int j = 0; j < 8; j++) {
-        float sum_x2 = 0;
-        for (int l = 0; l < 32; l++) sum_x2 += x[32 * j + l] * x[32 * j + l];
-        const float av_x = sqrtf(__fdiv_rn(sum_x2, 32.0f));  // IEEE sqrt: __fsqrt_rn is the native approximation here
-        for (int l = 0; l < 32; l++) w[l] = av_x + fabsf(x[32 * j + l]);
-        scales[j] = qkx2_fit<31, 15>(x + 32 * j, w, L + 32 * j, &mins[j], -0.5f);
-        if (scales[j] > max_scale) max_scale = scales[j];
-        if (mins[j] > max_min) max_min = mins[j];
+    uint8_t * o = out + i * (TYPE == T_Q4_K ? 144 : 176);
+    if (j == 0) {
+        uint32_t h[4] = {(uint32_t) dh | ((uint32_t) mh << 16), 0, 0, 0};
+#pragma unroll
+        for (int k = 0; k < 12; k++) h[1 + k / 4] |= (uint32_t) sb[k] << (8 * (k & 3));
+        put(o, make_uint4(h[0], h[1], h[2], h[3]));
     }
-    uint8_t sb[12];
-    uint16_t dh, mh;
-    pack_scale_min_k4(scales, mins, max_scale, max_min, sb, dh, mh);
-    for (int j = 0; j < 8; j++) {
-        int sc, m;
-        scale_min_k4(j, sb, sc, m);
-        const float d = h2f(dh) * (float) sc;
-        if (d == 0.0f) continue;  // the fit's codes stay, as in ggml
-        const float dm = h2f(mh) * (float) m;
-        for (int l = 0; l < 32; l++) {
-            int q = near_int(__fdiv_rn(x[32 * j + l] + dm, d));
-            L[32 * j + l] = (uint8_t) (q < 0 ? 0 : (q > 31 ? 31 : q));
+    uint8_t * ql = o + 16;
+    if constexpr (TYPE == T_Q5_K) {
+        uint32_t hb[8];
+#pragma unroll
+        for (int q = 0; q < 8; q++) {
+            hb[q] = ((c[q] >> 4) & 0x01010101u) << j;
+            c[q] &= 0x0F0F0F0Fu;
+            for (int s = 1; s < 8; s <<= 1) hb[q] |= __shfl_xor(hb[q], s, 64);
         }
+        if (j == 0) put(o + 16, make_uint4(hb[0], hb[1], hb[2], hb[3]));
+        if (j == 1) put(o + 32, make_uint4(hb[4], hb[5], hb[6], hb[7]));
+        ql = o + 48;
     }
-    uint8_t * o = out + i * 176;
-    o[0] = (uint8_t) dh;
-    o[1] = (uint8_t) (dh >> 8);
-    o[2] = (uint8_t) mh;
-    o[3] = (uint8_t) (mh >> 8);
-    for (int j = 0; j < 12; j++) o[4 + j] = sb[j];
-    uint8_t * qh = o + 16;
-    uint8_t * ql = o + 48;
-    for (int l = 0; l < 32; l++) qh[l] = 0;
-    for (int c = 0; c < 4; c++) {
-        for (int l = 0; l < 32; l++) {
-            int l1 = L[64 * c + l], l2 = L[64 * c + 32 + l];
-            if (l1 > 15) {
-                l1 -= 16;
-                qh[l] |= (uint8_t) (1u << (2 * c));
-            }
-            if (l2 > 15) {
-                l2 -= 16;
-                qh[l] |= (uint8_t) (2u << (2 * c));
-            }
-            ql[32 * c + l] = (uint8_t) (l1 | (l2 << 4));
-        }
+    // bytes of sub-blocks 2c (low nibbles) and 2c + 1 (high): the even lane writes the first 16, the odd the rest
+    const bool odd = j & 1;
+    uint32_t r[4];
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+        const uint32_t got = __shfl_xor(odd ? c[q] : c[4 + q], 1, 64);
+        r[q] = odd ? got | (c[4 + q] << 4) : c[q] | (got << 4);
     }
+    put(ql + 16 * j, make_uint4(r[0], r[1], r[2], r[3]));
 }
 
 // ggml make_qx_quants(16, 32, x, L, rmse_type = 1, no weights): the symmetric scale of 16 values
 // with codes l + 32, l in [-32, 31], refined over 18 candidate inverse scales by the x^2-weighted
-// least-squares fit. L receives the codes (0..63).
-__device__ float qx_fit16(const float * x, uint8_t * L) {
+// least-squares fit. The codes are those of l_iscale (zero: the values are all zero, and the codes 0).
+__device__ __forceinline__ float qx_fit16(const float (&x)[16], float & l_iscale, bool & zero) {
 #pragma clang fp contract(off)
     constexpr int nmax = 32;
     float max = 0, amax = 0;
+#pragma unroll
     for (int i = 0; i < 16; i++) {
         const float ax = fabsf(x[i]);
         if (ax > amax) {
@@ -283,102 +306,100 @@ __device__ float qx_fit16(const float * x, uint8_t * L) {
             max = x[i];
         }
     }
-    if (amax < 1e-15f) {  // GROUP_MAX_EPS
-        for (int i = 0; i < 16; i++) L[i] = 0;
-        return 0.0f;
-    }
-    float iscale = __fdiv_rn((float) -nmax, max);
-    float sumlx = 0, suml2 = 0;
-    for (int i = 0; i < 16; i++) {
-        int l = near_int(iscale * x[i]);
-        l = l < -nmax ? -nmax : (l > nmax - 1 ? nmax - 1 : l);
-        L[i] = (uint8_t) (l + nmax);
-        const float w = x[i] * x[i];
-        sumlx += w * x[i] * (float) l;
-        suml2 += w * (float) l * (float) l;
-    }
-    float scale = suml2 != 0.0f ? __fdiv_rn(sumlx, suml2) : 0.0f;
-    float best = scale * sumlx;
-    for (int is = -9; is <= 9; is++) {
-        if (is == 0) continue;
-        iscale = __fdiv_rn(-((float) nmax + 0.1f * (float) is), max);
-        sumlx = suml2 = 0;
+    zero = amax < 1e-15f;  // GROUP_MAX_EPS
+    l_iscale = 0.0f;
+    if (zero) return 0.0f;
+    float scale = 0, best = 0;
+    for (int k = -1; k < 19; k++) {  // k = -1: the plain scale; then is = -9 .. 9
+        const int is = k - 9;
+        if (k >= 0 && is == 0) continue;
+        const float iscale = __fdiv_rn(k < 0 ? (float) -nmax : -((float) nmax + 0.1f * (float) is), max);
+        float sumlx = 0, suml2 = 0;
+#pragma unroll
         for (int i = 0; i < 16; i++) {
-            int l = near_int(iscale * x[i]);
-            l = l < -nmax ? -nmax : (l > nmax - 1 ? nmax - 1 : l);
+            const float l = code<-nmax, nmax - 1>(iscale * x[i]);
             const float w = x[i] * x[i];
-            sumlx += w * x[i] * (float) l;
-            suml2 += w * (float) l * (float) l;
+            sumlx += w * x[i] * l;
+            suml2 += w * l * l;
         }
-        if (suml2 > 0 && sumlx * sumlx > best * suml2) {
-            for (int i = 0; i < 16; i++) {
-                int l = near_int(iscale * x[i]);
-                L[i] = (uint8_t) (nmax + (l < -nmax ? -nmax : (l > nmax - 1 ? nmax - 1 : l)));
-            }
-            scale = __fdiv_rn(sumlx, suml2);
+        if (k < 0 || (suml2 > 0 && sumlx * sumlx > best * suml2)) {
+            l_iscale = iscale;
+            scale = k >= 0 || suml2 != 0.0f ? __fdiv_rn(sumlx, suml2) : 0.0f;
             best = scale * sumlx;
         }
     }
     return scale;
 }
 
-// ggml quantize_row_q6_K_ref, one thread per 256-value super-block, written in ggml's 210-byte
-// block_q6_K {ql[128], qh[64], scales[16] int8, fp16 d}: 16 sub-block fits, int8 scales against
-// the largest-magnitude one (iscale = -128 / max), codes recomputed against the rounded scales.
-__global__ void k_enc_q6_K(const float * __restrict__ xall, uint8_t * __restrict__ out, int64_t nblocks) {
+// ggml quantize_row_q6_K_ref, sixteen lanes per 256-value super-block, a 16-value sub-block each,
+// written in ggml's 210-byte block_q6_K {ql[128], qh[64], scales[16] int8, fp16 d}: the sub-block fits,
+// int8 scales against the largest-magnitude one (iscale = -128 / max), codes recomputed against
+// the rounded scales.
+__global__ __launch_bounds__(256) void k_enc_q6_K(const float * __restrict__ xall, uint8_t * __restrict__ out,
+                                                  int64_t nblocks) {
 #pragma clang fp contract(off)
-    const int64_t i = (int64_t) blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= nblocks) return;
-    const float * x = xall + i * QKK;
-    uint8_t * o = out + i * 210;
-    uint8_t L[QKK];
-    float scales[16];
-    float max_scale = 0, max_abs_scale = 0;
-    for (int ib = 0; ib < 16; ib++) {
-        const float sc = qx_fit16(x + 16 * ib, L + 16 * ib);
-        scales[ib] = sc;
-        if (fabsf(sc) > max_abs_scale) {
-            max_abs_scale = fabsf(sc);
-            max_scale = sc;
+    const int64_t t = (int64_t) blockIdx.x * blockDim.x + threadIdx.x, i = t >> 4;
+    if (i >= nblocks) return;  // whole 16-lane groups
+    const int j = (int) (t & 15), lane0 = (threadIdx.x & 63) & ~15;
+    float x[16];
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+        const float4 v = get4(xall + t * 16 + 4 * q);
+        x[4 * q] = v.x, x[4 * q + 1] = v.y, x[4 * q + 2] = v.z, x[4 * q + 3] = v.w;
+    }
+    float l_iscale;
+    bool zero;
+    const float scale = qx_fit16(x, l_iscale, zero);
+    // the scale of largest magnitude, ties to the lowest sub-block
+    float max_abs = fabsf(scale) > 0 ? fabsf(scale) : 0.0f, max_scale = max_abs > 0 ? scale : 0.0f;
+    int at = max_abs > 0 ? j : 16;
+    for (int o = 1; o < 16; o <<= 1) {
+        const float a2 = __shfl_xor(max_abs, o, 64), s2 = __shfl_xor(max_scale, o, 64);
+        const int at2 = __shfl_xor(at, o, 64);
+        if (a2 > max_abs || (a2 == max_abs && at2 < at)) {
+            max_abs = a2;
+            max_scale = s2;
+            at = at2;
         }
     }
-    if (max_abs_scale < 1e-15f) {  // an all-zero block
-        for (int j = 0; j < 210; j++) o[j] = 0;
-        return;
-    }
+    const bool none = max_abs < 1e-15f;  // an all-zero block: all bytes zero
     const float iscale = __fdiv_rn(-128.0f, max_scale);
-    const uint16_t dh = f2h_exact(__fdiv_rn(1.0f, iscale));
-    int8_t sc8[16];
-    for (int ib = 0; ib < 16; ib++) {
-        const int v = near_int(iscale * scales[ib]);
-        sc8[ib] = (int8_t) (v < 127 ? v : 127);
-    }
-    for (int j = 0; j < 16; j++) {
-        const float d = h2f(dh) * (float) sc8[j];
-        if (d == 0.0f) continue;
-        for (int ii = 0; ii < 16; ii++) {
-            int l = near_int(__fdiv_rn(x[16 * j + ii], d));
-            l = l < -32 ? -32 : (l > 31 ? 31 : l);
-            L[16 * j + ii] = (uint8_t) (l + 32);
+    const uint16_t dh = none ? 0 : f2h_exact(__fdiv_rn(1.0f, iscale));
+    const int sv = near_int(iscale * scale);
+    const int sc = none ? 0 : (int) (int8_t) (sv < 127 ? sv : 127);
+    const float d = h2f(dh) * (float) sc;
+    uint32_t c[4];  // codes, 4 to a word
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+        c[q] = 0;
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            const float v = x[4 * q + e];
+            float l = code<-32, 31>(d == 0.0f ? l_iscale * v : __fdiv_rn(v, d)) + 32.0f;
+            if (none || (d == 0.0f && zero)) l = 0.0f;  // d == 0: the fit's codes stay, as in ggml
+            c[q] |= (uint32_t) (int) l << (8 * e);
         }
     }
-    uint8_t * ql = o;
-    uint8_t * qh = o + 128;
-    for (int h = 0; h < 2; h++) {
-        const uint8_t * Lh = L + 128 * h;
-        for (int l = 0; l < 32; l++) {
-            ql[64 * h + l] = (uint8_t) ((Lh[l] & 0xF) | ((Lh[l + 64] & 0xF) << 4));
-            ql[64 * h + 32 + l] = (uint8_t) ((Lh[l + 32] & 0xF) | ((Lh[l + 96] & 0xF) << 4));
-            qh[32 * h + l] = (uint8_t) ((Lh[l] >> 4) | ((Lh[l + 32] >> 4) << 2) | ((Lh[l + 64] >> 4) << 4) |
-                                        ((Lh[l + 96] >> 4) << 6));
-        }
+    // ql byte l < 64 of a half: values l (low nibble) and l + 64 (high), four sub-blocks on; qh byte l < 32:
+    // the top bits of values l, l + 32, l + 64, l + 96, two sub-blocks apart
+    const int h = j >> 3, s = j & 7;
+    uint32_t lo[4], hi[4];
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+        const uint32_t o4 = __shfl_xor(c[q], 4, 64);
+        lo[q] = (c[q] & 0x0F0F0F0Fu) | ((o4 & 0x0F0F0F0Fu) << 4);
+        const uint32_t tb = (c[q] >> 4) & 0x03030303u;
+        const int at0 = lane0 + 8 * h + (s & 1);
+        hi[q] = __shfl(tb, at0, 64) | (__shfl(tb, at0 + 2, 64) << 2) | (__shfl(tb, at0 + 4, 64) << 4) |
+                (__shfl(tb, at0 + 6, 64) << 6);
     }
-    for (int j = 0; j < 16; j++) o[192 + j] = (uint8_t) sc8[j];
-    o[208] = (uint8_t) dh;
-    o[209] = (uint8_t) (dh >> 8);
+    uint8_t * o = out + i * 210;
+    if (s < 4) put(o + 64 * h + 16 * s, make_uint4(lo[0], lo[1], lo[2], lo[3]));
+    else if (s < 6) put(o + 128 + 32 * h + 16 * (s - 4), make_uint4(hi[0], hi[1], hi[2], hi[3]));
+    o[192 + j] = (uint8_t) (int8_t) sc;
+    if (j == 15) put(o + 208, dh);
 }
 
-// f32 -> f16 rows (ggml_quantize_chunk for F16: round to nearest even).
 __global__ void k_enc_f16(const float * __restrict__ x, uint16_t * __restrict__ out, int64_t n) {
     const int64_t i = (int64_t) blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) out[i] = f2h_exact(x[i]);
@@ -667,11 +688,11 @@ void launch_encode(int type, const float * src, int64_t nrows, int64_t k, void *
     const int64_t nb = nrows * (k / (int64_t) block_elems(type));
     if (nb == 0) return;
     switch (type) {
-        case T_Q8_0: k_enc_q8_0<<<nblk(nb, 128), 128, 0, s>>>(src, (uint8_t *) dst, nb); break;
-        case T_Q4_0: k_enc_q4_0<<<nblk(nb, 128), 128, 0, s>>>(src, (uint8_t *) dst, nb); break;
-        case T_Q4_K: k_enc_q4_K<<<nblk(nb, 64), 64, 0, s>>>(src, (uint8_t *) dst, nb); break;
-        case T_Q5_K: k_enc_q5_K<<<nblk(nb, 64), 64, 0, s>>>(src, (uint8_t *) dst, nb); break;
-        case T_Q6_K: k_enc_q6_K<<<nblk(nb, 64), 64, 0, s>>>(src, (uint8_t *) dst, nb); break;
+        case T_Q8_0: k_enc_q8_0<<<nblk(nb * 8, 256), 256, 0, s>>>(src, (uint8_t *) dst, nb); break;
+        case T_Q4_0: k_enc_q4_0<<<nblk(nb * 8, 256), 256, 0, s>>>(src, (uint8_t *) dst, nb); break;
+        case T_Q4_K: k_enc_kq<T_Q4_K><<<nblk(nb * 8, 256), 256, 0, s>>>(src, (uint8_t *) dst, nb); break;
+        case T_Q5_K: k_enc_kq<T_Q5_K><<<nblk(nb * 8, 256), 256, 0, s>>>(src, (uint8_t *) dst, nb); break;
+        case T_Q6_K: k_enc_q6_K<<<nblk(nb * 16, 256), 256, 0, s>>>(src, (uint8_t *) dst, nb); break;
         case T_F16: k_enc_f16<<<nblk(nb, 256), 256, 0, s>>>(src, (uint16_t *) dst, nb); break;
         default: fail("encode: unsupported type " + std::to_string(type));
     }

@@ -100,3 +100,25 @@ def test_activation_kats(gops):
             continue
         assert to_np(got)[0].tobytes().hex() == k["hex"], name
 
+
+
+@pytest.mark.parametrize("t", ["q8_0", "q4_0", "q4_K", "q5_K", "q6_K"])
+def test_weight_encoders_edge_values(gops, orc, t):
+    """Blocks where the lane exchanges can go wrong, byte for byte: ties of the largest magnitude with
+    either sign first, constant and zero sub-blocks beside others, one large value, all-positive and
+    all-negative sub-blocks, tiny and large magnitudes; one block per row, so the grid ends inside a
+    wavefront."""
+    rng = np.random.default_rng(7)
+    x = (rng.standard_normal((11, 256)) * 0.02).astype(np.float32)
+    x[0, 5], x[0, 9], x[0, 40], x[0, 37] = 1.0, -1.0, -1.0, 1.0
+    x[1] = 0.0
+    x[2, :32], x[2, 64:96] = 0.25, 0.0
+    x[3] = np.abs(x[3])
+    x[4] = -np.abs(x[4])
+    x[5, 255] = 30.0
+    x[6] *= 1e-12
+    x[7] *= 1e4
+    x[8, 16:32], x[8, 128:] = 0.0, 0.0
+    x[9] = np.tile(np.array([0.5, -0.5], np.float32), 128)
+    got = to_np(gops.quantize(torch.from_numpy(x).cuda(), t))
+    assert np.array_equal(got, orc.quantize(x, t))
