@@ -12,7 +12,8 @@
 // Attention is HBM-bound by the K/V stream. Both kernels split the keys: grid = (split, KV head
 // [, query row]), each workgroup streams one contiguous slice of its KV head's rows once and
 // serves all G = H/Hkv query heads that share it. One query row (decode) runs k_attn_decode on the
-// matrix cores; prompt rows run k_attn_split (D/8 lanes cover one 2*D-byte row; pass 1 forms the
+// matrix cores; several rows run k_attn_prompt (attn_prompt.hip); head sizes and masks it does not
+// take run k_attn_split (D/8 lanes cover one 2*D-byte row; pass 1 forms the
 // scores with v_dot2_f32_f16 into LDS, pass 2 the slice's max and exp-sum, pass 3 P.V). A merge
 // (k_attn_merge, or the prologue of the GEMV that reads the attention row) combines the splits'
 // (max, sum, partial output) exactly as one online softmax would.
@@ -517,7 +518,50 @@ __global__ __launch_bounds__(256) void k_attn_merge(const float * __restrict__ p
     }
 }
 
+// The same for at most 8 splits: D / 4 threads per (query row, head), every split's partial loaded at once,
+// no LDS (512 x 32 rows of 4 splits: 16.9 us with a workgroup each, 8.2 so).
+constexpr int kMergeFew = 8;
+template <int D>
+__global__ __launch_bounds__(256) void k_attn_merge_few(const float * __restrict__ part_o, const float2 * __restrict__ part_ml,
+                                                        float * __restrict__ out, int nsplit, int64_t n) {
+    constexpr int Q = D / 4;
+    const int64_t t = (int64_t) blockIdx.x * 256 + threadIdx.x, sh = t / Q;
+    const int d4 = (int) (t % Q);
+    if (sh >= n) return;
+    float2 ml[kMergeFew];
+    f4_t o[kMergeFew];
+#pragma unroll
+    for (int i = 0; i < kMergeFew; i++) {
+        const int64_t at = sh * nsplit + min(i, nsplit - 1);
+        ml[i] = part_ml[at];
+        o[i] = *reinterpret_cast<const f4_t *>(part_o + at * D + 4 * d4);
+    }
+    float M = -INFINITY;
+#pragma unroll
+    for (int i = 0; i < kMergeFew; i++) M = fmaxf(M, ml[i].x);
+    float L = 0.0f;
+    f4_t r{};
+#pragma unroll
+    for (int i = 0; i < kMergeFew; i++) {
+        if (i >= nsplit || ml[i].x == -INFINITY) continue;
+        const float w = __expf(ml[i].x - M);
+        L += w * ml[i].y;
+        r += w * o[i];
+    }
+    const f4_t z{};
+    *reinterpret_cast<f4_t *>(out + sh * D + 4 * d4) = L == 0.0f ? z : r / L;
+}
+
 // ------------------------------------------------------------------------------- dispatch
+
+bool attn_prompt_fits(int D, int Sq, int H, int Hkv);
+int attn_prompt_max_split(int Sq, int H, int Hkv, int n_kv);
+AttnPlan attn_plan_prompt(int Sq, int H, int Hkv, int n_kv);
+void launch_attn_prompt(const float * q, int64_t q_h, int64_t q_s, const void * k, int64_t k_h, int64_t k_j,
+                        const void * v, int64_t v_h, int64_t v_j, const void * mask, int64_t m_s, int pos0, int D, int Sq,
+                        int H, int Hkv, int n_kv, float scale, float * out, float * part_o, float2 * part_ml,
+                        const AttnPlan & p, void * bits, hipStream_t s);
+size_t attn_prompt_bits(int Sq, int H, int Hkv, int n_kv);
 
 AttnPlan attn_plan(int Sq, int Hkv, int n_kv) {
     int nsplit = (n_kv + 63) / 64;
@@ -647,9 +691,13 @@ void launch_attn_decode(const float * q, int64_t q_h, const void * k, int64_t k_
 }
 
 size_t attn_workspace(int Sq, int H, int Hkv, int Dv, int n_kv) {
-    const AttnPlan p = attn_plan(Sq, Hkv, n_kv);
-    return align256((size_t) Sq * H * p.nsplit * Dv * sizeof(float)) +
-           align256((size_t) Sq * H * p.nsplit * sizeof(float2));
+    int nsplit = attn_plan(Sq, Hkv, n_kv).nsplit;
+    size_t bits = 0;
+    if (Sq > 1 && H % Hkv == 0) {
+        nsplit = std::max(nsplit, attn_prompt_max_split(Sq, H, Hkv, n_kv));
+        bits = attn_prompt_bits(Sq, H, Hkv, n_kv);
+    }
+    return bits + align256((size_t) Sq * H * nsplit * Dv * sizeof(float)) + align256((size_t) Sq * H * nsplit * sizeof(float2));
 }
 
 template <int D>
@@ -694,6 +742,19 @@ void launch_attn_split(const float * q, int64_t q_h, int64_t q_s, const void * k
     else run_split<256>(G, q, q_h, q_s, kk, k_h, k_j, vv, v_h, v_j, mm, m_s, Sq, H, Hkv, n_kv, scale, po, pml, p, n_kv_dev, s);
 }
 
+// The splits of n (query row, head) pairs combined into out [n][D].
+static void launch_merge(int D, const float * po, const float2 * pml, float * out, int nsplit, int64_t n, hipStream_t s) {
+    if (nsplit <= kMergeFew) {
+        const unsigned grid = (unsigned) ((n * (D / 4) + 255) / 256);
+        if (D == 64) k_attn_merge_few<64><<<grid, 256, 0, s>>>(po, pml, out, nsplit, n);
+        else k_attn_merge_few<128><<<grid, 256, 0, s>>>(po, pml, out, nsplit, n);
+    } else {
+        if (D == 64) k_attn_merge<64><<<(unsigned) n, 256, 0, s>>>(po, pml, out, nsplit);
+        else k_attn_merge<128><<<(unsigned) n, 256, 0, s>>>(po, pml, out, nsplit);
+    }
+    check_launch("flash_attn merge");
+}
+
 void launch_flash_attn(const float * q, int64_t q_h, int64_t q_s, const void * k, int64_t k_h, int64_t k_j,
                        const void * v, int64_t v_h, int64_t v_j, const void * mask, int64_t m_s, float * out, int D,
                        int Dv, int Sq, int H, int Hkv, int n_kv, float scale, void * ws, size_t ws_size,
@@ -717,6 +778,17 @@ void launch_flash_attn(const float * q, int64_t q_h, int64_t q_s, const void * k
         if (D == 64) k_attn_merge<64><<<(unsigned) H, 256, 0, s>>>(po, pml, out, nsplit);
         else k_attn_merge<128><<<(unsigned) H, 256, 0, s>>>(po, pml, out, nsplit);
         check_launch("flash_attn merge");
+        return;
+    }
+    if (attn_prompt_fits(D, Sq, H, Hkv) && (!mask || n_kv >= 4) && k_j < (1 << 24) && v_j < (1 << 24)) {
+        const AttnPlan pp = attn_plan_prompt(Sq, H, Hkv, n_kv);
+        const size_t bits = attn_prompt_bits(Sq, H, Hkv, n_kv);  // the workspace: bits, then the partials
+        po = (float *) ((uint8_t *) ws + bits);
+        pml = (float2 *) ((uint8_t *) po + align256((size_t) Sq * H * pp.nsplit * Dv * sizeof(float)));
+        launch_attn_prompt(q, q_h, q_s, k, k_h, k_j, v, v_h, v_j, mask, m_s, -1, D, Sq, H, Hkv, n_kv, scale,
+                           pp.nsplit == 1 ? out : nullptr, po, pml, pp, ws, s);
+        if (pp.nsplit == 1) return;
+        launch_merge(D, po, pml, out, pp.nsplit, (int64_t) Sq * H, s);
         return;
     }
     launch_attn_split(q, q_h, q_s, k, k_h, k_j, v, v_h, v_j, mask, m_s, D, Sq, H, Hkv, n_kv, scale, po, pml, p,

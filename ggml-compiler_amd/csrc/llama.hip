@@ -47,6 +47,13 @@ void launch_swiglu_q8(const float * g, const float * u, int64_t ld, int64_t n, i
                       hipStream_t s);
 void launch_rope_kv(float * qkv, int64_t ld, const int32_t * pos, int S, int H, int Hkv, int D, float base,
                     void * cache, int64_t ctx, hipStream_t s);
+bool attn_prompt_fits(int D, int Sq, int H, int Hkv);
+int attn_prompt_max_split(int Sq, int H, int Hkv, int n_kv);
+AttnPlan attn_plan_prompt(int Sq, int H, int Hkv, int n_kv);
+void launch_attn_prompt(const float * q, int64_t q_h, int64_t q_s, const void * k, int64_t k_h, int64_t k_j,
+                        const void * v, int64_t v_h, int64_t v_j, const void * mask, int64_t m_s, int pos0, int D, int Sq,
+                        int H, int Hkv, int n_kv, float scale, float * out, float * part_o, float2 * part_ml,
+                        const AttnPlan & p, void * bits, hipStream_t s);
 void launch_merge_q8(const float * part_o, const float2 * part_ml, int nsplit, int Sq, int H, int D, float * out,
                      void * act, hipStream_t s);
 void launch_causal_mask(void * mask, int S, int n_kv, int pos0, hipStream_t s);
@@ -196,9 +203,10 @@ struct Llama {
         act_b = DevBuf(act_layout(c.wtype, max_prompt, widest).total);
         size_t po = 0, pml = 0;
         for (int S = 1; S <= max_prompt; S++) {
-            const AttnPlan p = attn_plan(S, c.n_head_kv, c.max_ctx);
-            po = std::max(po, (size_t) S * c.n_head * p.nsplit * c.head_dim * 4);
-            pml = std::max(pml, (size_t) S * c.n_head * p.nsplit * 8);
+            const int nsplit = S > 1 ? attn_prompt_max_split(S, c.n_head, c.n_head_kv, c.max_ctx)
+                                     : attn_plan(S, c.n_head_kv, c.max_ctx).nsplit;
+            po = std::max(po, (size_t) S * c.n_head * nsplit * c.head_dim * 4);
+            pml = std::max(pml, (size_t) S * c.n_head * nsplit * 8);
         }
         // One token runs on the decode-row GEMVs when every projection's K fits them: QKV and
         // gate/up are then packed in row pairs (rope pairs, gate/up pairs) for their epilogues.
@@ -231,7 +239,7 @@ struct Llama {
         }
         part_o = DevBuf(po);
         part_ml = DevBuf(pml);
-        mask = DevBuf((size_t) max_prompt * c.max_ctx * 2);
+        mask = DevBuf((size_t) c.max_ctx * 2);
         positions = DevBuf((size_t) max_prompt * 4);
         tok_in = DevBuf((size_t) max_prompt * 4);
         logits = DevBuf((size_t) c.n_vocab * 4);
@@ -492,9 +500,15 @@ struct Llama {
         norm_mul_mat(L.attn_norm, L.qkv, xs, S, false, qkv.as<float>(), qkv_dim);
         launch_rope_kv(qkv.as<float>(), qkv_dim, pos_dev, S, c.n_head, c.n_head_kv, c.head_dim, c.rope_base, kvl,
                        c.max_ctx, stream);
-        launch_attn_split(qkv.as<float>(), c.head_dim, qkv_dim, kvl, kv_h, c.head_dim, kvl + (size_t) c.n_head_kv * kv_h,
-                          kv_h, c.head_dim, mask_dev, n_kv, c.head_dim, S, c.n_head, c.n_head_kv, n_kv, scale,
-                          part_o.as<float>(), part_ml.as<float2>(), plan, n_kv_dev, stream);
+        const uint16_t * vl = kvl + (size_t) c.n_head_kv * kv_h;
+        if (S > 1)  // the rows' positions end at n_kv - 1: causal, no mask tensor
+            launch_attn_prompt(qkv.as<float>(), c.head_dim, qkv_dim, kvl, kv_h, c.head_dim, vl, kv_h, c.head_dim, nullptr, 0,
+                               n_kv - S, c.head_dim, S, c.n_head, c.n_head_kv, n_kv, scale, nullptr, part_o.as<float>(),
+                               part_ml.as<float2>(), plan, nullptr, stream);
+        else
+            launch_attn_split(qkv.as<float>(), c.head_dim, qkv_dim, kvl, kv_h, c.head_dim, vl, kv_h, c.head_dim, mask_dev,
+                              n_kv, c.head_dim, S, c.n_head, c.n_head_kv, n_kv, scale, part_o.as<float>(),
+                              part_ml.as<float2>(), plan, n_kv_dev, stream);
         launch_merge_q8(part_o.as<float>(), part_ml.as<float2>(), plan.nsplit, S, c.n_head, c.head_dim, nullptr,
                         act_b.p, stream);
         mul_mat(L.wo, act_b.p, S, xs, c.n_embd, xs);
@@ -535,8 +549,8 @@ struct Llama {
             check_hip(hipMemcpyAsync(positions.p, p.data(), n * 4, hipMemcpyHostToDevice, stream), "positions");
             check_hip(hipMemcpyAsync(xs, x_in, row_bytes, hipMemcpyHostToDevice, stream), "x");
             const int n_kv = pos0 + n;
-            launch_causal_mask(mask.p, n, n_kv, pos0, stream);
-            const AttnPlan plan = attn_plan(n, c.n_head_kv, n_kv);
+            if (n == 1) launch_causal_mask(mask.p, n, n_kv, pos0, stream);
+            const AttnPlan plan = prompt_plan(n, n_kv);
             for (int l = first; l < first + count; l++)
                 prompt_layer(l, n, positions.as<int32_t>(), n_kv, nullptr, mask.p, plan,
                              mid ? mid_dev.as<float>() + (size_t) (l - first) * n * c.n_embd : nullptr);
@@ -557,14 +571,18 @@ struct Llama {
             check_hip(hipMemcpyAsync(positions.p, p.data(), S * 4, hipMemcpyHostToDevice, stream), "positions");
             check_hip(hipMemcpyAsync(tok_in.p, tokens + i, S * 4, hipMemcpyHostToDevice, stream), "tokens");
             const int n_kv = pos + S;
-            launch_causal_mask(mask.p, S, n_kv, pos, stream);
-            forward(S, tok_in.as<int32_t>(), positions.as<int32_t>(), n_kv, nullptr, mask.p,
-                    attn_plan(S, c.n_head_kv, n_kv));
+            if (S == 1) launch_causal_mask(mask.p, S, n_kv, pos, stream);
+            forward(S, tok_in.as<int32_t>(), positions.as<int32_t>(), n_kv, nullptr, mask.p, prompt_plan(S, n_kv));
             check_hip(hipStreamSynchronize(stream), "prefill");
             pos += S;
         }
         if (logits_host)
             check_hip(hipMemcpy(logits_host, logits.p, (size_t) c.n_vocab * 4, hipMemcpyDeviceToHost), "logits");
+    }
+
+    // The attention plan of a prompt chunk of S rows, the last of which sees n_kv keys.
+    AttnPlan prompt_plan(int S, int n_kv) const {
+        return S > 1 ? attn_plan_prompt(S, c.n_head, c.n_head_kv, n_kv) : attn_plan(S, c.n_head_kv, n_kv);
     }
 
     // The attention plan of a decode step that sees at most n_kv keys.

@@ -103,3 +103,40 @@ def test_decode_row_with_holes_in_the_mask(gops, orc, H, Hkv):
     m16 = orc.fp32_to_fp16(mask)
     out = _run(gops, q, kc, vc, m16, n_kv, 1 / np.sqrt(D))
     assert orc.parity(out, orc.flash_attn_ext(q, kc, vc, m16, 1 / np.sqrt(D))) < TOL
+
+
+@pytest.mark.parametrize("H,Hkv,D", [(4, 4, 64), (14, 2, 64), (8, 2, 128), (12, 4, 128), (16, 2, 128)])
+@pytest.mark.parametrize("Sq,n_kv", [(2, 2), (5, 67), (9, 64), (17, 300), (65, 65), (129, 256), (200, 1111)])
+@pytest.mark.parametrize("masked", [True, False])
+def test_prompt_rows(gops, orc, H, Hkv, D, Sq, n_kv, masked):
+    """Prompt attention on the matrix cores: 1, 2 and 4 row groups (up to 32, up to 64, more rows of a KV
+    head), partial row tiles and key blocks, heads per KV head that do not divide a tile, one and
+    several key splits; causal masks whose blocks are empty, full and partial, and no mask. f32 sums over
+    n_kv keys and weights kept to 22 bits: 1e-5 holds with room."""
+    q, kc, vc, m16 = _case(orc, H, Hkv, Sq, n_kv, D, n_kv + 5, seed=50)
+    out = _run(gops, q, kc, vc, m16 if masked else None, n_kv, D ** -0.5)
+    ref = orc.flash_attn_ext(q, kc[:, :n_kv], vc[:, :n_kv], m16 if masked else None, D ** -0.5)
+    assert orc.parity(out, ref) < 1e-5
+
+
+def test_prompt_rows_mask_values(gops, orc):
+    """Finite mask values (added to the scores), -inf keys scattered through blocks, a row that sees no key
+    (zeros), rows whose first visible key is far in, a mask with a wider row stride; scores spread over
+    a hundred powers of two (the reference exponent moves block by block)."""
+    H, Hkv, D, Sq, n_kv = 8, 2, 128, 33, 523
+    q, kc, vc, _ = _case(orc, H, Hkv, Sq, n_kv, D, n_kv, seed=51)
+    rng = np.random.default_rng(3)
+    m = rng.standard_normal((Sq, n_kv)).astype(np.float32) * 2
+    m[rng.random((Sq, n_kv)) < 0.3] = -np.inf
+    m[4] = -np.inf
+    m[7, :500] = -np.inf
+    m[8] += np.linspace(-40, 30, n_kv)
+    m16 = orc.fp32_to_fp16(m)
+    wide = np.zeros((Sq, n_kv + 13), np.uint16)
+    wide[:, :n_kv] = m16
+    out = to_np(gops.flash_attn_ext(torch.from_numpy(q).cuda(), torch.from_numpy(kc.view(np.float16)).cuda(),
+                                    torch.from_numpy(vc.view(np.float16)).cuda(),
+                                    torch.from_numpy(wide.view(np.float16)).cuda(), 0.3, n_kv=n_kv))
+    ref = orc.flash_attn_ext(q, kc, vc, m16, 0.3)
+    assert np.all(out.reshape(Sq, -1)[4] == 0.0)
+    assert orc.parity(out, ref) < 1e-5
