@@ -321,3 +321,37 @@ def test_gemm_kquant_k_groups(gops, orc, t, M, N, K):
     x = orc.normal((M, K), seed=42)
     y = to_np(gops.mul_mat(qw, torch.from_numpy(x).cuda()))
     assert orc.parity(y, orc.mul_mat(raw, t, x, K)) < 1e-5
+
+
+@pytest.mark.parametrize("t", ["q4_0", "q8_0"])
+@pytest.mark.parametrize("M,N,K", [(9, 31, 32), (33, 65, 96), (40, 200, 1056), (33, 6200, 160), (97, 16300, 288),
+                                   (300, 9100, 160), (129, 24800, 96)])
+def test_gemm_k_groups(gops, orc, t, M, N, K):
+    """Each tile of the GEMM at its edges: 32 x 32 tiles in eight K groups (fewer blocks than a step, a step that
+    starts early) and in four, 128 x 128 in two groups (one group a chunk short) and without, each also onto a
+    residual. Block sums are exact, so only f32 sums of K / 32 terms differ: 1e-5 covers any order of them."""
+    raw, qw = _weight(gops, orc, t, N, K, 43)
+    x = orc.normal((M, K), seed=44)
+    ref = orc.mul_mat(raw, t, x, K)
+    xd = torch.from_numpy(x).cuda()
+    assert orc.parity(to_np(gops.mul_mat(qw, xd)), ref) < 1e-5
+    res = orc.normal((M, N), seed=45)
+    act = gops.quantize_act(t, xd)
+    y = to_np(gops.mul_mat_q(qw, act, M, res=torch.from_numpy(res).cuda()))
+    assert orc.parity(y, ref + res) < 1e-5
+
+
+@pytest.mark.parametrize("M,N", [(9, 64), (33, 6200), (300, 9100), (129, 24800)])
+def test_gemm_infinite_weight_scale(gops, orc, M, N):
+    """A block with an infinite scale gives isum * inf, not a NaN from inf - inf: the sign of its block sum."""
+    K = 64
+    raw, _ = _weight(gops, orc, "q8_0", N, K, 46)
+    raw = raw.copy().reshape(N, -1)
+    raw[5, 0:2] = [0x00, 0x7C]  # d of row 5's first block: +inf
+    qw = gops.QuantWeight.from_ggml(torch.from_numpy(raw), "q8_0", K)
+    x = torch.ones((M, K), device="cuda")
+    q = raw[5, 2:34].view(np.int8)
+    assert q.astype(np.int64).sum() != 0
+    y = to_np(gops.mul_mat(qw, x))
+    assert np.all(y[:, 5] == np.sign(q.astype(np.int64).sum()) * np.inf)
+    assert np.all(np.isfinite(np.delete(y, 5, axis=1)))
