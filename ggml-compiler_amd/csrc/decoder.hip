@@ -37,7 +37,9 @@ __global__ __launch_bounds__(256) void k_rmsnorm_q8(const float * __restrict__ x
     rmsnorm_q8_row(x + row * ldx, n, w, eps, codes + (int64_t) row * n, meta + (int64_t) row * (n / 32));
 }
 
-// silu(g) * u over rows of n (g, u at row strides), quantized to Q8_0.
+// silu(g) * u over rows of n (g, u at row strides), quantized to Q8_0. PAIRS: g holds a row's (g, u) pairs side by
+// side (the decoder's packed gate / up order) and u is not read.
+template <bool PAIRS>
 __global__ void k_swiglu_q8(const float * __restrict__ g, const float * __restrict__ u, int64_t ld, int n, int rows,
                             int8_t * __restrict__ codes, float2 * __restrict__ meta) {
     const int64_t t = (int64_t) blockIdx.x * blockDim.x + threadIdx.x;
@@ -45,9 +47,16 @@ __global__ void k_swiglu_q8(const float * __restrict__ g, const float * __restri
     if (t >= (int64_t) rows * per) return;  // whole 8-lane groups
     const int row = (int) (t / per);
     const int e = (int) (t % per) * 4;
-    const float4 a = *reinterpret_cast<const float4 *>(g + row * ld + e);
-    const float4 b = *reinterpret_cast<const float4 *>(u + row * ld + e);
-    float4 v;
+    float4 a, b, v;
+    if constexpr (PAIRS) {
+        const float4 p = *reinterpret_cast<const float4 *>(g + row * ld + 2 * e);
+        const float4 q = *reinterpret_cast<const float4 *>(g + row * ld + 2 * e + 4);
+        a = make_float4(p.x, p.z, q.x, q.z);
+        b = make_float4(p.y, p.w, q.y, q.w);
+    } else {
+        a = *reinterpret_cast<const float4 *>(g + row * ld + e);
+        b = *reinterpret_cast<const float4 *>(u + row * ld + e);
+    }
     v.x = a.x / (1.0f + expf(-a.x)) * b.x;
     v.y = a.y / (1.0f + expf(-a.y)) * b.y;
     v.z = a.z / (1.0f + expf(-a.z)) * b.z;
@@ -55,38 +64,59 @@ __global__ void k_swiglu_q8(const float * __restrict__ g, const float * __restri
     q8_block_store(v, codes + (int64_t) row * n + (e & ~31), meta + (int64_t) row * (n / 32) + e / 32, (e / 4) & 7);
 }
 
-// NEOX rope (n_dims = D) of the H q heads and Hkv k heads of each fused QKV row [q | k | v], q in
-// place, roped k and v written as f16 into the cache rows pos[s]: cache [2*Hkv][ctx][D], K heads
-// first. One thread per rotation pair (q and k) or per value pair (v).
-__global__ void k_rope_kv(float * __restrict__ qkv, int64_t ld, const int32_t * __restrict__ pos, int S, int H,
+// NEOX rope (n_dims = D) of the H q heads and Hkv k heads of each fused QKV row [q | k | v], q into the row of
+// dst (ld), roped k and v written as f16 into the cache rows pos[s]: cache [2*Hkv][ctx][D], K heads
+// first. PAIRS: src rows hold a head's rotation pairs (i, i + D/2) side by side (the decoder's packed order; v
+// as it is); else src is dst. One thread per rotation index and kRopeHeads heads, or per value pair (v).
+// The angle (the power as i multiplications, cosf, sinf) bounds it, not the bytes: a thread per head and pair
+// took 14.6 us at 500 rows of 32 + 8 + 8 heads of 128, after 7.8 us of putting the packed columns back; 8.0 so.
+constexpr int kRopeHeads = 8;
+template <bool PAIRS>
+__global__ void k_rope_kv(const float * src, float * dst, int64_t ld, const int32_t * __restrict__ pos, int S, int H,
                           int Hkv, int D, float theta_scale, uint16_t * __restrict__ cache, int64_t ctx) {
-    const int half = D / 2;
-    const int per_s = (H + 2 * Hkv) * half;
+    const int half = D / 2, groups = (H + Hkv + kRopeHeads - 1) / kRopeHeads;
+    const int per_s = (groups + Hkv) * half;
     const int64_t t = (int64_t) blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= (int64_t) S * per_s) return;
     const int s = (int) (t / per_s);
     const int r = (int) (t % per_s);
-    const int h = r / half, i = r % half;
+    const int g = r / half, i = r % half;
     const int p = pos[s];
     if (p < 0 || p >= ctx) return;
-    float * row = qkv + s * ld;
-    if (h < H + Hkv) {
+    const float * row = src + s * ld;
+    if (g < groups) {
         float theta = (float) p;
         for (int k = 0; k < i; k++) theta *= theta_scale;
         const float c = cosf(theta), sn = sinf(theta);
-        float * xr = row + h * D;
-        const float x0 = xr[i], x1 = xr[i + half];
-        const float y0 = x0 * c - x1 * sn, y1 = x0 * sn + x1 * c;
-        if (h < H) {
-            xr[i] = y0;
-            xr[i + half] = y1;
-        } else {
-            uint16_t * kr = cache + ((int64_t) (h - H) * ctx + p) * D;
-            kr[i] = f2h(y0);
-            kr[i + half] = f2h(y1);
+        float xa[kRopeHeads], xb[kRopeHeads];
+#pragma unroll
+        for (int e = 0; e < kRopeHeads; e++) {
+            const float * xr = row + min(g * kRopeHeads + e, H + Hkv - 1) * D;
+            if constexpr (PAIRS) {
+                const float2 x = *reinterpret_cast<const float2 *>(xr + 2 * i);
+                xa[e] = x.x, xb[e] = x.y;
+            } else {
+                xa[e] = xr[i], xb[e] = xr[i + half];
+            }
+        }
+#pragma unroll
+        for (int e = 0; e < kRopeHeads; e++) {
+            const int h = g * kRopeHeads + e;
+            if (h >= H + Hkv) break;
+            const float x0 = xa[e], x1 = xb[e];
+            const float y0 = x0 * c - x1 * sn, y1 = x0 * sn + x1 * c;
+            if (h < H) {
+                float * yr = dst + s * ld + h * D;
+                yr[i] = y0;
+                yr[i + half] = y1;
+            } else {
+                uint16_t * kr = cache + ((int64_t) (h - H) * ctx + p) * D;
+                kr[i] = f2h(y0);
+                kr[i + half] = f2h(y1);
+            }
         }
     } else {  // v head hv: values 2i, 2i+1
-        const int hv = h - H - Hkv;
+        const int hv = g - groups;
         const float * vr = row + (H + Hkv + hv) * D;
         uint16_t * dr = cache + ((int64_t) (Hkv + hv) * ctx + p) * D;
         const uint32_t pair = f2h(vr[2 * i]) | ((uint32_t) f2h(vr[2 * i + 1]) << 16);
@@ -147,17 +177,6 @@ __global__ void k_embed_rope(int type, const uint8_t * __restrict__ tab, int64_t
         for (int k = 0; k < t; k++) theta *= theta_scale;
         cs[t] = make_float2(cosf(theta), sinf(theta));
     }
-}
-
-// dst[r][map[c]] = src[r][c] for S rows of n columns: a mul_mat result whose weight rows were
-// packed in another order, back in the weight's own row order.
-__global__ void k_scatter_cols(const float * __restrict__ src, int64_t lds, float * __restrict__ dst, int64_t ldd,
-                               const int32_t * __restrict__ map, int S, int n) {
-    const int64_t t = (int64_t) blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= (int64_t) S * n) return;
-    const int64_t r = t / n;
-    const int c = (int) (t % n);
-    dst[r * ldd + map[c]] = src[r * lds + c];
 }
 
 // mask[s][j] = 0 for j <= pos0 + s, -inf after (f16), j < n_kv.
@@ -230,16 +249,26 @@ void launch_rmsnorm_q8(const float * x, int64_t ldx, const float * w, float eps,
 void launch_swiglu_q8(const float * g, const float * u, int64_t ld, int64_t n, int64_t rows, void * act,
                       hipStream_t s) {
     const ActLayout L = act_layout(T_Q4_0, rows, n);
-    k_swiglu_q8<<<nblk(rows * n / 4, 256), 256, 0, s>>>(g, u, ld, (int) n, (int) rows, (int8_t *) act,
-                                                        (float2 *) ((uint8_t *) act + L.meta));
+    k_swiglu_q8<false><<<nblk(rows * n / 4, 256), 256, 0, s>>>(g, u, ld, (int) n, (int) rows, (int8_t *) act,
+                                                               (float2 *) ((uint8_t *) act + L.meta));
     check_launch("swiglu_q8");
 }
 
-void launch_rope_kv(float * qkv, int64_t ld, const int32_t * pos, int S, int H, int Hkv, int D, float base,
-                    void * cache, int64_t ctx, hipStream_t s) {
+// The same of rows of 2 n values, (g, u) pairs.
+void launch_swiglu_q8_pairs(const float * gu, int64_t ld, int64_t n, int64_t rows, void * act, hipStream_t s) {
+    const ActLayout L = act_layout(T_Q4_0, rows, n);
+    k_swiglu_q8<true><<<nblk(rows * n / 4, 256), 256, 0, s>>>(gu, nullptr, ld, (int) n, (int) rows, (int8_t *) act,
+                                                              (float2 *) ((uint8_t *) act + L.meta));
+    check_launch("swiglu_q8");
+}
+
+// src: the QKV rows in the decoder's packed order, or null (dst's own rows, in place).
+void launch_rope_kv(const float * src, float * dst, int64_t ld, const int32_t * pos, int S, int H, int Hkv, int D,
+                    float base, void * cache, int64_t ctx, hipStream_t s) {
     const float theta_scale = powf(base, -2.0f / (float) D);
-    const int64_t n = (int64_t) S * (H + 2 * Hkv) * (D / 2);
-    k_rope_kv<<<nblk(n, 256), 256, 0, s>>>(qkv, ld, pos, S, H, Hkv, D, theta_scale, (uint16_t *) cache, ctx);
+    const int64_t n = (int64_t) S * ((H + Hkv + kRopeHeads - 1) / kRopeHeads + Hkv) * (D / 2);
+    if (src) k_rope_kv<true><<<nblk(n, 256), 256, 0, s>>>(src, dst, ld, pos, S, H, Hkv, D, theta_scale, (uint16_t *) cache, ctx);
+    else k_rope_kv<false><<<nblk(n, 256), 256, 0, s>>>(dst, dst, ld, pos, S, H, Hkv, D, theta_scale, (uint16_t *) cache, ctx);
     check_launch("rope_kv");
 }
 
@@ -262,12 +291,6 @@ void launch_embed_rope(int type, const void * tab, int64_t nrows, int64_t D, con
     k_embed_rope<<<nblk(n, 256), 256, 0, s>>>(type, (const uint8_t *) tab, nrows, (int) D, idx, x, pos, half,
                                              theta_scale, (float2 *) cs);
     check_launch("embed_rope");
-}
-
-void launch_scatter_cols(const float * src, int64_t lds, float * dst, int64_t ldd, const int32_t * map, int S, int n,
-                         hipStream_t s) {
-    k_scatter_cols<<<nblk((int64_t) S * n, 256), 256, 0, s>>>(src, lds, dst, ldd, map, S, n);
-    check_launch("scatter_cols");
 }
 
 void launch_causal_mask(void * mask, int S, int n_kv, int pos0, hipStream_t s) {

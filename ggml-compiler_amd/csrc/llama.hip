@@ -45,8 +45,9 @@ void launch_rmsnorm_q8(const float * x, int64_t ldx, const float * w, float eps,
                        hipStream_t s);
 void launch_swiglu_q8(const float * g, const float * u, int64_t ld, int64_t n, int64_t rows, void * act,
                       hipStream_t s);
-void launch_rope_kv(float * qkv, int64_t ld, const int32_t * pos, int S, int H, int Hkv, int D, float base,
-                    void * cache, int64_t ctx, hipStream_t s);
+void launch_swiglu_q8_pairs(const float * gu, int64_t ld, int64_t n, int64_t rows, void * act, hipStream_t s);
+void launch_rope_kv(const float * src, float * dst, int64_t ld, const int32_t * pos, int S, int H, int Hkv, int D,
+                    float base, void * cache, int64_t ctx, hipStream_t s);
 bool attn_prompt_fits(int D, int Sq, int H, int Hkv);
 int attn_prompt_max_split(int Sq, int H, int Hkv, int n_kv);
 AttnPlan attn_plan_prompt(int Sq, int H, int Hkv, int n_kv);
@@ -59,8 +60,6 @@ void launch_merge_q8(const float * part_o, const float2 * part_ml, int nsplit, i
 void launch_causal_mask(void * mask, int S, int n_kv, int pos0, hipStream_t s);
 void launch_move_rows(const void * src, void * dst, const int32_t * map, int64_t rows, int64_t row_bytes, bool scatter,
                       hipStream_t s);
-void launch_scatter_cols(const float * src, int64_t lds, float * dst, int64_t ldd, const int32_t * map, int S, int n,
-                         hipStream_t s);
 AttnPlan attn_plan_decode(int D, int H, int G, int max_ctx, int max_split);
 bool attn_decode_fits(int D, int G);
 void launch_attn_decode(const float * q, int64_t q_h, const void * k, int64_t k_h, int64_t k_j, const void * v,
@@ -132,7 +131,7 @@ struct Llama {
     DevBuf attn_row;           // its output when it runs unsplit
     DevBuf rope_cs;            // the decode step's rotation table (cos, sin) per rotation index
     bool prefetch = false;     // attention's spare CUs read the next weights ahead (GCQ_DECODE_PREFETCH=1: on)
-    DevBuf ytmp;         // a prompt chunk's mul_mat result in packed row order
+    DevBuf ytmp;         // a prompt chunk's QKV rows in packed order
     int pos = 0;
     // The captured decode step, one graph per bucket of kKvBucket KV lengths (step_graph).
     static constexpr int kKvBucket = 32;
@@ -235,7 +234,7 @@ struct Llama {
                 set_perm(L.qkv, pq);
                 set_perm(L.gate_up, pg);
             }
-            ytmp = DevBuf((size_t) max_prompt * std::max<int64_t>(qkv_dim, 2 * (int64_t) c.n_ff) * 4);
+            ytmp = DevBuf((size_t) max_prompt * qkv_dim * 4);
         }
         part_o = DevBuf(po);
         part_ml = DevBuf(pml);
@@ -333,18 +332,11 @@ struct Llama {
         check_hip(hipMemcpy(host, (t.perm.p ? tmp : raw).p, nbytes, hipMemcpyDeviceToHost), "get_weight");
     }
 
+    // Columns of y in the weight's packed row order.
     void mul_mat(int ti, const void * act, int64_t S, float * y, int64_t ldy, const float * res) {
         const Tensor & t = tensors[ti];
-        float * out = y;
-        int64_t ldo = ldy;
-        if (t.perm.p) {  // rows packed in pairs: compute in packed order, then put columns back
-            require(res == nullptr, "mul_mat: residual on a row-paired weight");
-            out = ytmp.as<float>();
-            ldo = t.rows;
-        }
-        if (S <= 8) launch_gemv(t.type, t.buf.p, t.rows, t.cols, act, S, out, ldo, stream, res);
-        else launch_gemm(t.type, t.buf.p, t.rows, t.cols, act, S, out, ldo, stream, res);
-        if (t.perm.p) launch_scatter_cols(out, ldo, y, ldy, t.perm.as<int32_t>(), (int) S, (int) t.rows, stream);
+        if (S <= 8) launch_gemv(t.type, t.buf.p, t.rows, t.cols, act, S, y, ldy, stream, res);
+        else launch_gemm(t.type, t.buf.p, t.rows, t.cols, act, S, y, ldy, stream, res);
     }
 
     RowArgs row_args(int ti) const {
@@ -497,9 +489,10 @@ struct Llama {
         const int64_t kv_h = (int64_t) c.max_ctx * c.head_dim;
         const Layer & L = layers[l];
         uint16_t * kvl = kv_layer(l);
-        norm_mul_mat(L.attn_norm, L.qkv, xs, S, false, qkv.as<float>(), qkv_dim);
-        launch_rope_kv(qkv.as<float>(), qkv_dim, pos_dev, S, c.n_head, c.n_head_kv, c.head_dim, c.rope_base, kvl,
-                       c.max_ctx, stream);
+        // QKV and gate / up packed in row pairs (fused): their readers take the columns in that order
+        norm_mul_mat(L.attn_norm, L.qkv, xs, S, false, (fused ? ytmp : qkv).as<float>(), qkv_dim);
+        launch_rope_kv(fused ? ytmp.as<float>() : nullptr, qkv.as<float>(), qkv_dim, pos_dev, S, c.n_head, c.n_head_kv,
+                       c.head_dim, c.rope_base, kvl, c.max_ctx, stream);
         const uint16_t * vl = kvl + (size_t) c.n_head_kv * kv_h;
         if (S > 1)  // the rows' positions end at n_kv - 1: causal, no mask tensor
             launch_attn_prompt(qkv.as<float>(), c.head_dim, qkv_dim, kvl, kv_h, c.head_dim, vl, kv_h, c.head_dim, nullptr, 0,
@@ -514,7 +507,8 @@ struct Llama {
         mul_mat(L.wo, act_b.p, S, xs, c.n_embd, xs);
         if (mid) check_hip(hipMemcpyAsync(mid, xs, (size_t) S * c.n_embd * 4, hipMemcpyDeviceToDevice, stream), "mid");
         norm_mul_mat(L.ffn_norm, L.gate_up, xs, S, false, gu.as<float>(), 2 * (int64_t) c.n_ff);
-        launch_swiglu_q8(gu.as<float>(), gu.as<float>() + c.n_ff, 2 * (int64_t) c.n_ff, c.n_ff, S, act_b.p, stream);
+        if (fused) launch_swiglu_q8_pairs(gu.as<float>(), 2 * (int64_t) c.n_ff, c.n_ff, S, act_b.p, stream);
+        else launch_swiglu_q8(gu.as<float>(), gu.as<float>() + c.n_ff, 2 * (int64_t) c.n_ff, c.n_ff, S, act_b.p, stream);
         mul_mat(L.down, act_b.p, S, xs, c.n_embd, xs);
     }
 

@@ -79,6 +79,20 @@ def test_prefill_and_decode_match_oracle(gops, orc, wtype, n_prompt):
     assert m.position == n_prompt + 6
 
 
+@pytest.mark.parametrize("H,Hkv,D", [(12, 2, 64), (7, 1, 128), (6, 6, 128)])
+def test_prompt_rope_head_groups(gops, orc, H, Hkv, D):
+    """The prompt's rope takes 8 heads per thread from the packed QKV order: 14, 8 and 12 heads of 64 and 128
+    (a part group, a whole one, both), V heads after them."""
+    from ggml_compiler_amd.llm import LlamaConfig
+
+    cfg = LlamaConfig(n_layer=1, n_embd=768, n_head=H, n_head_kv=Hkv, head_dim=D, n_ff=544, n_vocab=500, max_ctx=64,
+                      wtype=2, rms_eps=1e-5, rope_base=10000.0)
+    m, o, _ = _models(cfg, seed=4)
+    for n in (3, 17):
+        prompt = orc.ids(n, seed=6 + n, vocab=cfg.n_vocab).tolist()
+        assert orc.parity(m.prefill(prompt), o.forward(prompt)) < TOL_LM
+
+
 def test_device_generate_equals_host_loop(gops):
     """The on-device generate loop makes the tokens the host loop makes (test_llm.py:178-201)."""
     from ggml_compiler_amd.llm import Generator
