@@ -234,6 +234,30 @@ __global__ __launch_bounds__(256) void k_step_end(const float * __restrict__ log
     }
 }
 
+// A step's or prompt chunk's small inputs as kernel arguments or from pinned host memory, and its results into
+// pinned host memory: a copy through pageable memory is a host round trip of its own (a decode step with its
+// logits and token read by the host took 164 us of which the GPU worked 95: a pageable upload, a
+// wait, two pageable downloads, 30-50 us each).
+__global__ void k_set_state(StepState * st, StepState v) { *st = v; }
+
+__global__ void k_prompt_in(const int32_t * __restrict__ host, int32_t * __restrict__ tok, int32_t * __restrict__ pos,
+                            int pos0, int n) {
+    const int t = blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= n) return;
+    tok[t] = host[t];
+    pos[t] = pos0 + t;
+}
+
+// n logits (0: none) and the state to host memory.
+__global__ void k_step_out(const float * __restrict__ logits, float * __restrict__ host, int n, const StepState * __restrict__ st,
+                           StepState * __restrict__ host_st) {
+    const int t = blockIdx.x * blockDim.x + threadIdx.x;
+    if (4 * t + 3 < n) *reinterpret_cast<float4 *>(host + 4 * t) = *reinterpret_cast<const float4 *>(logits + 4 * t);
+    else
+        for (int i = 4 * t; i < n; i++) host[i] = logits[i];
+    if (t == 0) *host_st = *st;
+}
+
 // ------------------------------------------------------------------------------ launchers
 
 static inline unsigned nblk(int64_t n, int t) { return (unsigned) ((n + t - 1) / t); }
@@ -306,6 +330,23 @@ void launch_step_end(const float * logits, int n, void * state, int32_t * out_to
     k_step_end<<<nblk(n, kArgmaxSlice), 256, 0, s>>>(logits, n, (StepState *) state, out_tokens, max_out, (float2 *) part,
                                               (unsigned int *) counter);
     check_launch("step_end");
+}
+
+void launch_set_state(void * state, int pos, int n_kv, int token, int step, hipStream_t s) {
+    k_set_state<<<1, 1, 0, s>>>((StepState *) state, StepState{pos, n_kv, token, step});
+    check_launch("set_state");
+}
+
+// tokens: pinned host memory; tok, pos: device rows of n.
+void launch_prompt_in(const int32_t * tokens, int32_t * tok, int32_t * pos, int pos0, int n, hipStream_t s) {
+    k_prompt_in<<<nblk(n, 256), 256, 0, s>>>(tokens, tok, pos, pos0, n);
+    check_launch("prompt_in");
+}
+
+// host, host_state: pinned host memory, 16-byte aligned.
+void launch_step_out(const float * logits, float * host, int n, const void * state, void * host_state, hipStream_t s) {
+    k_step_out<<<nblk((n + 3) / 4 + 1, 256), 256, 0, s>>>(logits, host, n, (const StepState *) state, (StepState *) host_state);
+    check_launch("step_out");
 }
 
 }  // namespace gcq

@@ -71,6 +71,9 @@ void launch_embed_rope(int type, const void * tab, int64_t nrows, int64_t D, con
                        const int32_t * pos, int head_dim, float base, void * cs, hipStream_t s);
 void launch_step_end(const float * logits, int n, void * state, int32_t * out_tokens, int max_out, void * part,
                      void * counter, hipStream_t s);
+void launch_set_state(void * state, int pos, int n_kv, int token, int step, hipStream_t s);
+void launch_prompt_in(const int32_t * tokens, int32_t * tok, int32_t * pos, int pos0, int n, hipStream_t s);
+void launch_step_out(const float * logits, float * host, int n, const void * state, void * host_state, hipStream_t s);
 
 int cu_count();
 
@@ -95,6 +98,22 @@ struct DevBuf {
     }
     ~DevBuf() {
         if (p) (void) hipFree(p);
+    }
+    template <class T> T * as() const { return reinterpret_cast<T *>(p); }
+};
+
+struct PinnedBuf {  // host memory that kernels read and write
+    void * p = nullptr;
+    PinnedBuf() = default;
+    explicit PinnedBuf(size_t bytes) { check_hip(hipHostMalloc(&p, std::max<size_t>(bytes, 256), hipHostMallocDefault), "hipHostMalloc"); }
+    PinnedBuf(const PinnedBuf &) = delete;
+    PinnedBuf & operator=(const PinnedBuf &) = delete;
+    PinnedBuf & operator=(PinnedBuf && o) noexcept {
+        std::swap(p, o.p);
+        return *this;
+    }
+    ~PinnedBuf() {
+        if (p) (void) hipHostFree(p);
     }
     template <class T> T * as() const { return reinterpret_cast<T *>(p); }
 };
@@ -132,6 +151,7 @@ struct Llama {
     DevBuf rope_cs;            // the decode step's rotation table (cos, sin) per rotation index
     bool prefetch = false;     // attention's spare CUs read the next weights ahead (GCQ_DECODE_PREFETCH=1: on)
     DevBuf ytmp;         // a prompt chunk's QKV rows in packed order
+    PinnedBuf host_tokens, host_logits, host_state;  // a chunk's tokens in; a call's logits and state out
     int pos = 0;
     // The captured decode step, one graph per bucket of kKvBucket KV lengths (step_graph).
     static constexpr int kKvBucket = 32;
@@ -243,6 +263,9 @@ struct Llama {
         tok_in = DevBuf((size_t) max_prompt * 4);
         logits = DevBuf((size_t) c.n_vocab * 4);
         state = DevBuf(sizeof(StepStateHost));
+        host_tokens = PinnedBuf((size_t) max_prompt * 4);
+        host_logits = PinnedBuf((size_t) c.n_vocab * 4);
+        host_state = PinnedBuf(sizeof(StepStateHost));
         out_tokens = DevBuf((size_t) c.max_ctx * 4);
         argmax_part = DevBuf(256 * sizeof(float2));
         counters = DevBuf(4096);
@@ -560,18 +583,17 @@ struct Llama {
                                           " tokens > max_ctx " + std::to_string(c.max_ctx));
         for (int i = 0; i < n; i += max_prompt) {
             const int S = std::min(max_prompt, n - i);
-            std::vector<int32_t> p(S);
-            for (int j = 0; j < S; j++) p[j] = pos + j;
-            check_hip(hipMemcpyAsync(positions.p, p.data(), S * 4, hipMemcpyHostToDevice, stream), "positions");
-            check_hip(hipMemcpyAsync(tok_in.p, tokens + i, S * 4, hipMemcpyHostToDevice, stream), "tokens");
+            std::memcpy(host_tokens.p, tokens + i, (size_t) S * 4);  // the last chunk has been waited for
+            launch_prompt_in(host_tokens.as<int32_t>(), tok_in.as<int32_t>(), positions.as<int32_t>(), pos, S, stream);
             const int n_kv = pos + S;
             if (S == 1) launch_causal_mask(mask.p, S, n_kv, pos, stream);
             forward(S, tok_in.as<int32_t>(), positions.as<int32_t>(), n_kv, nullptr, mask.p, prompt_plan(S, n_kv));
+            const bool out = logits_host && i + S == n;
+            if (out) results_out(true);
             check_hip(hipStreamSynchronize(stream), "prefill");
             pos += S;
+            if (out) std::memcpy(logits_host, host_logits.p, (size_t) c.n_vocab * 4);
         }
-        if (logits_host)
-            check_hip(hipMemcpy(logits_host, logits.p, (size_t) c.n_vocab * 4, hipMemcpyDeviceToHost), "logits");
     }
 
     // The attention plan of a prompt chunk of S rows, the last of which sees n_kv keys.
@@ -624,9 +646,11 @@ struct Llama {
         for (int b = 0; b * kKvBucket < upto; b++) (void) step_graph(std::min(upto, (b + 1) * kKvBucket));
     }
 
-    void set_state(int token) {
-        const StepStateHost st{pos, pos + 1, token, 0};
-        check_hip(hipMemcpyAsync(state.p, &st, sizeof st, hipMemcpyHostToDevice, stream), "state");
+    void set_state(int token) { launch_set_state(state.p, pos, pos + 1, token, 0, stream); }
+
+    // The state, and the logits if asked for, into pinned memory (there after the stream's next wait).
+    void results_out(bool with_logits) {
+        launch_step_out(logits.as<float>(), host_logits.as<float>(), with_logits ? c.n_vocab : 0, state.p, host_state.p, stream);
     }
 
     void decode(int32_t token, float * logits_host, int32_t * next) {
@@ -636,15 +660,11 @@ struct Llama {
         hipGraphExec_t step = step_graph(pos + 1);
         set_state(token);
         check_hip(hipGraphLaunch(step, stream), "graph launch");
+        if (logits_host || next) results_out(logits_host != nullptr);
         check_hip(hipStreamSynchronize(stream), "decode");
         pos += 1;
-        if (logits_host)
-            check_hip(hipMemcpy(logits_host, logits.p, (size_t) c.n_vocab * 4, hipMemcpyDeviceToHost), "logits");
-        if (next) {
-            StepStateHost st;
-            check_hip(hipMemcpy(&st, state.p, sizeof st, hipMemcpyDeviceToHost), "state");
-            *next = st.token;
-        }
+        if (logits_host) std::memcpy(logits_host, host_logits.p, (size_t) c.n_vocab * 4);
+        if (next) *next = host_state.as<StepStateHost>()->token;
     }
 
     void generate(int32_t first, int n_new, int32_t * out) {
