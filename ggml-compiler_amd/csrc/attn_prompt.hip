@@ -56,6 +56,9 @@ struct PromptArgs {
     int64_t m_s;
     const uint2 * bits;  // k_attn_mask_bits
     float scale2;   // |scale| * log2(e); negate: the scale is negative (Q's sign turns)
+    // A masked key's S becomes S mask_s + mask value * mask_m, its exponent mask_c2 times that: (1, 1 / |scale|, scale2),
+    // which leaves S as it is where the value is 0; or, where 1 / |scale| is out of range, (scale2, log2(e), 1).
+    float mask_s, mask_m, mask_c2;
     bool negate;
     int Sq, H, G, n_kv, pos0, blocks, nsplit;  // blocks: key blocks per split
     float * out, * part_o;
@@ -247,7 +250,7 @@ __global__ __launch_bounds__(64 * RW * KW, RW == 1 ? 1 : 2) void k_attn_prompt(c
         float mx = -INFINITY, c2 = a.scale2;  // a key's exponent is c2 S
         if (some) {
             asm volatile("");  // a branch: as selects this runs for every block
-            if (MODE == kMask) c2 = 1.0f;  // S becomes the exponent itself, mask value added
+            if (MODE == kMask) c2 = a.mask_c2;
             const uint16_t * mr = MODE == kMask ? a.mask + (int64_t) s * a.m_s : nullptr;
             const int left = a.n_kv - b * KB, seen = MODE == kCausal ? min(left, a.pos0 + s + 1 - b * KB) : left;
 #pragma unroll
@@ -268,7 +271,7 @@ __global__ __launch_bounds__(64 * RW * KW, RW == 1 ? 1 : 2) void k_attn_prompt(c
                         if constexpr (MODE == kMask) {
                             const float mv = h2f((uint16_t) (m >> (16 * r)));
                             drop = drop || mv == -INFINITY;
-                            S[t][e] = fmaf(S[t][e], a.scale2, mv * 1.44269504088896341f);
+                            S[t][e] = fmaf(S[t][e], a.mask_s, mv * a.mask_m);
                         }
                         S[t][e] = drop ? -INFINITY : S[t][e];
                     }
@@ -454,6 +457,9 @@ void launch_attn_prompt(const float * q, int64_t q_h, int64_t q_s, const void * 
     a.mask = (const uint16_t *) mask, a.m_s = m_s;
     a.scale2 = (float) (fabs((double) scale) * 1.4426950408889634074);
     a.negate = scale < 0.0f;
+    const double mag = fabs((double) scale);
+    if (mag >= 0x1p-60 && mag <= 0x1p60) a.mask_s = 1.0f, a.mask_m = (float) (1.0 / mag), a.mask_c2 = a.scale2;
+    else a.mask_s = a.scale2, a.mask_m = 1.44269504088896341f, a.mask_c2 = 1.0f;  // 0 and NaN too
     a.Sq = Sq, a.H = H, a.G = H / Hkv, a.n_kv = n_kv, a.pos0 = pos0, a.blocks = p.chunk / KB, a.nsplit = p.nsplit;
     a.out = out, a.part_o = part_o, a.part_ml = part_ml;
     const int mode = mask ? kMask : pos0 >= 0 ? kCausal : kAllKeys;
