@@ -12,7 +12,7 @@
 // Attention is HBM-bound by the K/V stream. Both kernels split the keys: grid = (split, KV head
 // [, query row]), each workgroup streams one contiguous slice of its KV head's rows once and
 // serves all G = H/Hkv query heads that share it. One query row (decode) runs k_attn_decode on the
-// matrix cores; several rows run k_attn_prompt (attn_prompt.hip); head sizes and masks it does not
+// matrix cores; several rows run k_attn_prompt (attn_prompt.hip); head sizes, masks and scales it does not
 // take run k_attn_split (D/8 lanes cover one 2*D-byte row; pass 1 forms the
 // scores with v_dot2_f32_f16 into LDS, pass 2 the slice's max and exp-sum, pass 3 P.V). A merge
 // (k_attn_merge, or the prologue of the GEMV that reads the attention row) combines the splits'
@@ -554,7 +554,7 @@ __global__ __launch_bounds__(256) void k_attn_merge_few(const float * __restrict
 
 // ------------------------------------------------------------------------------- dispatch
 
-bool attn_prompt_fits(int D, int Sq, int H, int Hkv);
+bool attn_prompt_fits(int D, int Sq, int H, int Hkv, float scale);
 int attn_prompt_max_split(int Sq, int H, int Hkv, int n_kv);
 AttnPlan attn_plan_prompt(int Sq, int H, int Hkv, int n_kv);
 void launch_attn_prompt(const float * q, int64_t q_h, int64_t q_s, const void * k, int64_t k_h, int64_t k_j,
@@ -780,7 +780,7 @@ void launch_flash_attn(const float * q, int64_t q_h, int64_t q_s, const void * k
         check_launch("flash_attn merge");
         return;
     }
-    if (attn_prompt_fits(D, Sq, H, Hkv) && (!mask || n_kv >= 4) && k_j < (1 << 24) && v_j < (1 << 24)) {
+    if (attn_prompt_fits(D, Sq, H, Hkv, scale) && (!mask || n_kv >= 4) && k_j < (1 << 24) && v_j < (1 << 24)) {
         const AttnPlan pp = attn_plan_prompt(Sq, H, Hkv, n_kv);
         const size_t bits = attn_prompt_bits(Sq, H, Hkv, n_kv);  // the workspace: bits, then the partials
         po = (float *) ((uint8_t *) ws + bits);

@@ -56,9 +56,7 @@ struct PromptArgs {
     int64_t m_s;
     const uint2 * bits;  // k_attn_mask_bits
     float scale2;   // |scale| * log2(e); negate: the scale is negative (Q's sign turns)
-    // A masked key's S becomes S mask_s + mask value * mask_m, its exponent mask_c2 times that: (1, 1 / |scale|, scale2),
-    // which leaves S as it is where the value is 0; or, where 1 / |scale| is out of range, (scale2, log2(e), 1).
-    float mask_s, mask_m, mask_c2;
+    float mask_m;   // 1 / |scale|: a masked key's S becomes S + mask value * mask_m, as it is where the value is 0
     bool negate;
     int Sq, H, G, n_kv, pos0, blocks, nsplit;  // blocks: key blocks per split
     float * out, * part_o;
@@ -247,10 +245,10 @@ __global__ __launch_bounds__(64 * RW * KW, RW == 1 ? 1 : 2) void k_attn_prompt(c
 #pragma unroll
             for (int t = 0; t < KT; t++)
                 S[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(*reinterpret_cast<const h8_t *>(kp + 32 * t * KP + 16 * c), qf[c], S[t], 0, 0, 0);
-        float mx = -INFINITY, c2 = a.scale2;  // a key's exponent is c2 S
+        const float c2 = a.scale2;  // a key's exponent is c2 S
+        float mx = -INFINITY;
         if (some) {
             asm volatile("");  // a branch: as selects this runs for every block
-            if (MODE == kMask) c2 = a.mask_c2;
             const uint16_t * mr = MODE == kMask ? a.mask + (int64_t) s * a.m_s : nullptr;
             const int left = a.n_kv - b * KB, seen = MODE == kCausal ? min(left, a.pos0 + s + 1 - b * KB) : left;
 #pragma unroll
@@ -271,7 +269,7 @@ __global__ __launch_bounds__(64 * RW * KW, RW == 1 ? 1 : 2) void k_attn_prompt(c
                         if constexpr (MODE == kMask) {
                             const float mv = h2f((uint16_t) (m >> (16 * r)));
                             drop = drop || mv == -INFINITY;
-                            S[t][e] = fmaf(S[t][e], a.mask_s, mv * a.mask_m);
+                            S[t][e] = fmaf(mv, a.mask_m, S[t][e]);
                         }
                         S[t][e] = drop ? -INFINITY : S[t][e];
                     }
@@ -409,9 +407,11 @@ void run(const PromptArgs & a, int Hkv, int mode, hipStream_t s) {
 
 }  // namespace
 
-// (A mask needs rows of at least four values: launch_attn_prompt.)
-bool attn_prompt_fits(int D, int Sq, int H, int Hkv) {
-    return (D == 64 || D == 128) && Sq > 1 && H % Hkv == 0 && (int64_t) Sq * (H / Hkv) < INT32_MAX;
+// (A mask needs rows of at least four values: launch_attn_prompt.) The scale's range: a dropped key's weight is
+// 2^(scale -inf), not 0 where the scale is 0, and a mask value is divided by the scale; k_attn_split takes the rest.
+bool attn_prompt_fits(int D, int Sq, int H, int Hkv, float scale) {
+    return (D == 64 || D == 128) && Sq > 1 && H % Hkv == 0 && (int64_t) Sq * (H / Hkv) < INT32_MAX &&
+           fabsf(scale) >= 0x1p-60f && fabsf(scale) <= 0x1p60f;
 }
 
 // Key splits: about 512 workgroups in all (two per CU), each split of at least two key blocks (no more for a
@@ -441,7 +441,7 @@ void launch_attn_prompt(const float * q, int64_t q_h, int64_t q_s, const void * 
                         const void * v, int64_t v_h, int64_t v_j, const void * mask, int64_t m_s, int pos0, int D, int Sq,
                         int H, int Hkv, int n_kv, float scale, float * out, float * part_o, float2 * part_ml,
                         const AttnPlan & p, void * bits, hipStream_t s) {
-    require(attn_prompt_fits(D, Sq, H, Hkv), "attn prompt: D 64 or 128, more than one query row");
+    require(attn_prompt_fits(D, Sq, H, Hkv, scale), "attn prompt: D 64 or 128, more than one query row, a scale within 2^-60 .. 2^60");
     require(p.chunk % KB == 0 && (int64_t) p.nsplit * p.chunk >= n_kv, "attn prompt: the splits must cover the keys");
     require(((int64_t) Sq * (H / Hkv) / 32 + 1) * Hkv * p.nsplit < INT32_MAX, "attn prompt: too many row tiles");
     require(!out || p.nsplit == 1, "attn prompt: several splits go to the merge");
@@ -457,9 +457,7 @@ void launch_attn_prompt(const float * q, int64_t q_h, int64_t q_s, const void * 
     a.mask = (const uint16_t *) mask, a.m_s = m_s;
     a.scale2 = (float) (fabs((double) scale) * 1.4426950408889634074);
     a.negate = scale < 0.0f;
-    const double mag = fabs((double) scale);
-    if (mag >= 0x1p-60 && mag <= 0x1p60) a.mask_s = 1.0f, a.mask_m = (float) (1.0 / mag), a.mask_c2 = a.scale2;
-    else a.mask_s = a.scale2, a.mask_m = 1.44269504088896341f, a.mask_c2 = 1.0f;  // 0 and NaN too
+    a.mask_m = (float) (1.0 / fabs((double) scale));
     a.Sq = Sq, a.H = H, a.G = H / Hkv, a.n_kv = n_kv, a.pos0 = pos0, a.blocks = p.chunk / KB, a.nsplit = p.nsplit;
     a.out = out, a.part_o = part_o, a.part_ml = part_ml;
     const int mode = mask ? kMask : pos0 >= 0 ? kCausal : kAllKeys;

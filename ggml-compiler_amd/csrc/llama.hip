@@ -48,7 +48,6 @@ void launch_swiglu_q8(const float * g, const float * u, int64_t ld, int64_t n, i
 void launch_swiglu_q8_pairs(const float * gu, int64_t ld, int64_t n, int64_t rows, void * act, hipStream_t s);
 void launch_rope_kv(const float * src, float * dst, int64_t ld, const int32_t * pos, int S, int H, int Hkv, int D,
                     float base, void * cache, int64_t ctx, hipStream_t s);
-bool attn_prompt_fits(int D, int Sq, int H, int Hkv);
 int attn_prompt_max_split(int Sq, int H, int Hkv, int n_kv);
 AttnPlan attn_plan_prompt(int Sq, int H, int Hkv, int n_kv);
 void launch_attn_prompt(const float * q, int64_t q_h, int64_t q_s, const void * k, int64_t k_h, int64_t k_j,

@@ -140,3 +140,21 @@ def test_prompt_rows_mask_values(gops, orc):
     ref = orc.flash_attn_ext(q, kc, vc, m16, 0.3)
     assert np.all(out.reshape(Sq, -1)[4] == 0.0)
     assert orc.parity(out, ref) < 1e-5
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("n_kv", [64, 67, 300])
+@pytest.mark.parametrize("masked", [True, False])
+@pytest.mark.parametrize("scale", [0.0, -0.0, 1e-40, 2.0 ** -61, -(2.0 ** -60), -0.1, -(2.0 ** 61), 2.0 ** 100])
+def test_prompt_rows_scales(gops, orc, D, n_kv, masked, scale):
+    """Every finite scale over several query rows: 0 gives the mean of the visible values, tiny ones too; negative
+    ones; huge ones the value of the best key. Whole-number q and k make the dot products exact, so the best keys (ties among
+    them) are the same ones in every order of the sums."""
+    H, Hkv, Sq = 8, 2, 9
+    rng = np.random.default_rng(n_kv)
+    q = rng.integers(-3, 4, (H, Sq, D)).astype(np.float32)
+    kc = orc.fp32_to_fp16(rng.integers(-3, 4, (Hkv, n_kv, D)).astype(np.float32))
+    _, _, vc, m16 = _case(orc, H, Hkv, Sq, n_kv, D, n_kv, seed=52)
+    m16 = m16 if masked else None
+    out = _run(gops, q, kc, vc, m16, n_kv, scale)
+    assert orc.parity(out, orc.flash_attn_ext(q, kc, vc, m16, scale)) < 1e-5
