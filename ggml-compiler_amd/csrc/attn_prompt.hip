@@ -245,7 +245,7 @@ __global__ __launch_bounds__(64 * RW * KW, RW == 1 ? 1 : 2) void k_attn_prompt(c
 #pragma unroll
             for (int t = 0; t < KT; t++)
                 S[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(*reinterpret_cast<const h8_t *>(kp + 32 * t * KP + 16 * c), qf[c], S[t], 0, 0, 0);
-        const float c2 = a.scale2;  // a key's exponent is c2 S
+        float c2 = a.scale2;  // a key's exponent is c2 S
         float mx = -INFINITY;
         if (some) {
             asm volatile("");  // a branch: as selects this runs for every block
@@ -286,6 +286,15 @@ __global__ __launch_bounds__(64 * RW * KW, RW == 1 ? 1 : 2) void k_attn_prompt(c
         R = Rn;
         // 2^(c2 S - R) with one rounding of the small difference, then the exact scale
         const float base = R == -INFINITY ? 0.0f : R;
+        // From 2^22 on R is c2 S rounded by up to a quarter and more: the largest S must be rounded alike.
+        if (__builtin_expect(__any(fabsf(base) >= 0x1p22f), 0)) {
+            asm volatile("");
+#pragma unroll
+            for (int t = 0; t < KT; t++)
+#pragma unroll
+                for (int e = 0; e < 16; e++) S[t][e] *= c2;
+            c2 = 1.0f;
+        }
 #pragma unroll
         for (int t = 0; t < KT; t++)
 #pragma unroll

@@ -145,7 +145,8 @@ def test_prompt_rows_mask_values(gops, orc):
 @pytest.mark.parametrize("D", [64, 128])
 @pytest.mark.parametrize("n_kv", [64, 67, 300])
 @pytest.mark.parametrize("masked", [True, False])
-@pytest.mark.parametrize("scale", [0.0, -0.0, 1e-40, 2.0 ** -61, -(2.0 ** -60), -0.1, -(2.0 ** 61), 2.0 ** 100])
+@pytest.mark.parametrize("scale", [0.0, -0.0, 1e-40, 2.0 ** -61, -(2.0 ** -60), -0.1, 1e5, -3e6, 7e7, 2.0 ** 31,
+                                   -(2.0 ** 45), 2.0 ** 60, -(2.0 ** 61), 2.0 ** 100])
 def test_prompt_rows_scales(gops, orc, D, n_kv, masked, scale):
     """Every finite scale over several query rows: 0 gives the mean of the visible values, tiny ones too; negative
     ones; huge ones the value of the best key. Whole-number q and k make the dot products exact, so the best keys (ties among
