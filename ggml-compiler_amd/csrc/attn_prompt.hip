@@ -356,6 +356,64 @@ __global__ __launch_bounds__(64 * RW * KW, RW == 1 ? 1 : 2) void k_attn_prompt(c
             for (int e = 0; e < 16; e++) O[t][e] = 0.0f;
     }
 
+    // An infinite V value: its product with P's remainder (0 or negative for most weights) has made a NaN of the sums.
+    // A wavefront whose sums are not all finite forms them again key by key, with the weights in f32.
+    float fin = 0.0f;
+#pragma unroll
+    for (int t = 0; t < D / 32; t++)
+#pragma unroll
+        for (int e = 0; e < 16; e++) fin = fmaf(O[t][e], 0.0f, fin);  // NaN if any is not finite
+    if (__builtin_expect(__any(fin != fin), 0)) {
+        asm volatile("");
+#pragma unroll
+        for (int t = 0; t < D / 32; t++)
+#pragma unroll
+            for (int e = 0; e < 16; e++) O[t][e] = 0.0f;
+        for (int bs = next(b0); bs < b1; bs = next(bs + 1)) {
+            const int j0 = bs * KB + (KW == 2 ? 32 * kw : 0);
+            int j1 = min(j0 + KB / KW, a.n_kv);
+            if (MODE == kCausal) j1 = min(j1, a.pos0 + s + 1);
+#pragma unroll 1
+            for (int j = j0; j < min(j0 + KB / KW, a.n_kv); j++) {
+                float x = 0.0f;  // lanes lr and lr + 32 hold the dims in halves
+#pragma unroll
+                for (int c = 0; c < D / 16; c++) {
+                    u4_t kf;
+                    __builtin_memcpy(&kf, kb + (int64_t) j * a.k_j + 16 * c + 8 * lk, 16);
+                    const u4_t qc = __builtin_bit_cast(u4_t, qf[c]);
+#pragma unroll
+                    for (int i = 0; i < 4; i++) {
+                        const uint32_t kw2 = kf[i], qw2 = qc[i];  // (a bit_cast of kf[i] itself takes element 0)
+                        x = __builtin_amdgcn_fdot2(__builtin_bit_cast(h2_t, kw2), __builtin_bit_cast(h2_t, qw2), x, false);
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+                x = xhalf_sum(x);
+                bool drop = j >= j1;
+                if constexpr (MODE == kMask) {
+                    const float mv = h2f(a.mask[(int64_t) s * a.m_s + j]);
+                    drop = drop || mv == -INFINITY;
+                    x = fmaf(mv, a.mask_m, x);
+                }
+                x *= a.scale2;
+                const float p = __builtin_amdgcn_exp2f(x - R) * kPScale;
+                if (drop || R == -INFINITY) continue;
+                const uint16_t * vj = vb + (int64_t) j * a.v_j + 4 * lk;
+#pragma unroll
+                for (int t = 0; t < D / 32; t++)
+#pragma unroll
+                    for (int i = 0; i < 4; i++) {
+                        u2_t w;
+                        __builtin_memcpy(&w, vj + 32 * t + 8 * i, 8);
+#pragma unroll
+                        for (int r = 0; r < 4; r++)
+                            O[t][4 * i + r] = fmaf(p, h2f((uint16_t) ((r < 2 ? w.x : w.y) >> (16 * (r & 1)))), O[t][4 * i + r]);
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
+            }
+        }
+    }
+
     if constexpr (KW == 2) {  // the two key halves: the second hands its sums to the first
         float * ex = reinterpret_cast<float *>(&L[0]) + (size_t) rw * 64 * (D / 2 + 2) + lane;
         static_assert(sizeof(L) >= (size_t) RW * 64 * (D / 2 + 2) * 4, "exchange fits");

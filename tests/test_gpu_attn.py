@@ -159,3 +159,29 @@ def test_prompt_rows_scales(gops, orc, D, n_kv, masked, scale):
     m16 = m16 if masked else None
     out = _run(gops, q, kc, vc, m16, n_kv, scale)
     assert orc.parity(out, orc.flash_attn_ext(q, kc, vc, m16, scale)) < 1e-5
+
+
+def _same_with_infinities(out, ref, tol):
+    for kind in (np.isnan, np.isposinf, np.isneginf):
+        assert np.array_equal(kind(out), kind(ref)), kind.__name__
+    f = np.isfinite(ref)
+    assert np.max(np.abs(out[f] - ref[f])) < tol * max(1.0, np.max(np.abs(ref[f])))
+
+
+@pytest.mark.parametrize("H,Hkv,D,Sq", [(8, 2, 64, 5), (8, 2, 128, 5), (8, 2, 128, 13), (8, 2, 64, 70), (8, 2, 128, 70)])
+@pytest.mark.parametrize("n_kv", [96, 1000])
+@pytest.mark.parametrize("masked", [True, False])
+def test_prompt_rows_infinite_values(gops, orc, H, Hkv, D, Sq, n_kv, masked):
+    """A V value that overflowed f16: every row that sees its key with any weight (e^-40 of the largest, too) gets that
+    infinity in its dim, a NaN where both signs meet, and no other dim or row changes; a key that a row does not see
+    does not count. A NaN in V alike."""
+    q, kc, vc, m16 = _case(orc, H, Hkv, Sq, n_kv, D, n_kv, seed=53)
+    m = np.zeros((Sq, n_kv), np.float32)
+    m[:, n_kv - Sq:] = np.where(np.arange(Sq)[None] <= np.arange(Sq)[:, None], 0, -np.inf)
+    m[:, 20] = -40
+    vc = vc.copy()
+    vc[0, 7, 3], vc[0, 20, 11], vc[0, n_kv - 2, 3] = 0x7C00, 0xFC00, 0xFC00  # +inf; -inf at the weight e^-40; -inf late
+    vc[1, 40, 30] = 0x7E00  # NaN
+    m16 = orc.fp32_to_fp16(m) if masked else None
+    out = _run(gops, q, kc, vc, m16, n_kv, D ** -0.5)
+    _same_with_infinities(out, orc.flash_attn_ext(q, kc, vc, m16, D ** -0.5), 1e-5)
