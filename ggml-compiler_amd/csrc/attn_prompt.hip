@@ -45,7 +45,7 @@ constexpr int VP = KB + 4;      // pitch of a V^T row (halves): 16 lanes' 8-byte
 // Up to these keys every block takes the mask: looking it over first costs a launch (129 rows x 256 keys, 14 / 2
 // heads of 64: 22.2 us with it, 18.9 without).
 constexpr int kBitsKeys = 512;
-constexpr float kPScale = 8192.0f;  // P's scale
+constexpr float kPScale = 32768.0f;  // P's scale
 
 struct PromptArgs {
     const float * q;
@@ -118,6 +118,7 @@ __global__ __launch_bounds__(64 * RW * KW, RW == 1 ? 1 : 2) void k_attn_prompt(c
     constexpr int KP = D + 8;                       // pitch of a K row (halves)
     constexpr int KL = KB * (D / 8) / NT;           // 16-byte K pieces per thread
     constexpr int VL = (D / 32) * (KB / 32) / NW;   // 4-key x 4-dim V tiles per lane
+    constexpr int NP = RW <= 2 ? 3 : 2;             // f16 parts of a weight
     struct Lds {
         _Float16 k[KB * KP];
         _Float16 v[D * VP];
@@ -236,15 +237,18 @@ __global__ __launch_bounds__(64 * RW * KW, RW == 1 ? 1 : 2) void k_attn_prompt(c
         bool some = b * KB + KB > a.n_kv;
         if constexpr (MODE == kCausal) some = some || b * KB + KB - 1 > a.pos0 + s_first;
         if constexpr (MODE == kMask) some = some || !bits || ((uint32_t) __builtin_amdgcn_readfirstlane((int) bits[b >> 5].y) >> (b & 31) & 1);
+        // Dots of D values: chains of two MFMAs, added in f32. A sum inside the MFMA is cut off, not rounded, against a
+        // growing accumulator (one chain of eight: 1.10 times the error of f32 dots, four chains 0.95).
         v16f S[KT];
         const _Float16 * kp = lds.k + (32 * (KW == 2 ? kw : 0) + lr) * KP + 8 * lk;
 #pragma unroll
-        for (int t = 0; t < KT; t++) S[t] = v16f{};
+        for (int t = 0; t < KT; t++) {
+            v16f A[4]{};
 #pragma unroll
-        for (int c = 0; c < D / 16; c++)
-#pragma unroll
-            for (int t = 0; t < KT; t++)
-                S[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(*reinterpret_cast<const h8_t *>(kp + 32 * t * KP + 16 * c), qf[c], S[t], 0, 0, 0);
+            for (int c = 0; c < D / 16; c++)
+                A[c % 4] = __builtin_amdgcn_mfma_f32_32x32x16_f16(*reinterpret_cast<const h8_t *>(kp + 32 * t * KP + 16 * c), qf[c], A[c % 4], 0, 0, 0);
+            S[t] = (A[0] + A[1]) + (A[2] + A[3]);
+        }
         float c2 = a.scale2;  // a key's exponent is c2 S
         float mx = -INFINITY;
         if (some) {
@@ -299,48 +303,45 @@ __global__ __launch_bounds__(64 * RW * KW, RW == 1 ? 1 : 2) void k_attn_prompt(c
         for (int t = 0; t < KT; t++)
 #pragma unroll
             for (int e = 0; e < 16; e++) S[t][e] = __builtin_amdgcn_exp2f(fmaf(S[t][e], c2, -base)) * kPScale;
-        // The block's sum of weights from zero, as P V below (one long chain of sums: 2.5e-7 off instead of 2.3e-7).
+        // The weights as NP f16 parts, each rounded to nearest. Two: the sum of weights is of what the parts hold, so that
+        // numerator and denominator see the same weights; three: all 24 bits.
         float ls[2] = {0.0f, 0.0f};
-        h8_t ph[2 * KT], pl[2 * KT];  // 16 keys each: k slot (lk, j) is key 16 c + 4 lk + j, or + 8 + 4 lk + j - 4
+        h8_t ph[NP][2 * KT];  // 16 keys each: k slot (lk, j) is key 16 c + 4 lk + j, or + 8 + 4 lk + j - 4
+        constexpr h2_t one = {(_Float16) 1.0f, (_Float16) 1.0f};
 #pragma unroll
         for (int c = 0; c < 2 * KT; c++)
 #pragma unroll
             for (int j = 0; j < 8; j += 2) {
-                const float p0 = S[c >> 1][8 * (c & 1) + j], p1 = S[c >> 1][8 * (c & 1) + j + 1];
-                ls[0] += p0;
-                ls[1] += p1;
-                // both parts rounded to nearest: truncated ones would leave P V low
-                const h2_t hi = {(_Float16) p0, (_Float16) p1};
-                const h2_t lo = {(_Float16) fmaf((float) hi.x, -1.0f, p0), (_Float16) fmaf((float) hi.y, -1.0f, p1)};
-                ph[c][j] = hi.x, ph[c][j + 1] = hi.y;
-                pl[c][j] = lo.x, pl[c][j + 1] = lo.y;
+                float p0 = S[c >> 1][8 * (c & 1) + j], p1 = S[c >> 1][8 * (c & 1) + j + 1];
+                if constexpr (NP == 3) ls[0] += p0, ls[1] += p1;
+#pragma unroll
+                for (int n = 0; n < NP; n++) {
+                    const h2_t w = {(_Float16) p0, (_Float16) p1};
+                    if constexpr (NP == 2) ls[n] = __builtin_amdgcn_fdot2(w, one, ls[n], false);
+                    p0 = fmaf((float) w.x, -1.0f, p0);
+                    p1 = fmaf((float) w.y, -1.0f, p1);
+                    ph[n][c][j] = w.x, ph[n][c][j + 1] = w.y;
+                }
             }
         l = fmaf(l, al, ls[0] + ls[1]);
-        // The block's P V from zero, then one multiply-add into the sums (with their rescaling): an f32 rounding
-        // per block there instead of one per 16 keys and part (n_kv = 4096: 3.6e-7 off instead of 2.5e-7).
+        // The block's P V from zero, its first part and the others in chains of their own, then one multiply-add into
+        // the sums (with their rescaling): few additions inside the MFMAs (as above), and one f32 rounding per block.
         const _Float16 * vp = lds.v + lr * VP + 32 * (KW == 2 ? kw : 0) + 4 * lk;
 #pragma unroll
-        for (int d2 = 0; d2 < D / 32; d2 += 2) {  // two at a time (all four leave no registers for the staged loads)
+        for (int d = 0; d < D / 32; d++) {  // one at a time (more leave no registers for the staged loads)
             __builtin_amdgcn_sched_barrier(0);
-            v16f T[2]{};
+            v16f T{}, Tl{};
 #pragma unroll
             for (int c = 0; c < 2 * KT; c++) {
-                h8_t vf[2];
+                const u2_t v0 = *reinterpret_cast<const u2_t *>(vp + 32 * d * VP + 16 * c);
+                const u2_t v1 = *reinterpret_cast<const u2_t *>(vp + 32 * d * VP + 16 * c + 8);
+                const h8_t vf = __builtin_bit_cast(h8_t, u4_t{v0.x, v0.y, v1.x, v1.y});
 #pragma unroll
-                for (int d = 0; d < 2; d++) {
-                    const u2_t v0 = *reinterpret_cast<const u2_t *>(vp + 32 * (d2 + d) * VP + 16 * c);
-                    const u2_t v1 = *reinterpret_cast<const u2_t *>(vp + 32 * (d2 + d) * VP + 16 * c + 8);
-                    vf[d] = __builtin_bit_cast(h8_t, u4_t{v0.x, v0.y, v1.x, v1.y});
-                }
-#pragma unroll
-                for (int d = 0; d < 2; d++) T[d] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf[d], pl[c], T[d], 0, 0, 0);
-#pragma unroll
-                for (int d = 0; d < 2; d++) T[d] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf[d], ph[c], T[d], 0, 0, 0);
+                for (int n = NP - 1; n > 0; n--) Tl = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf, ph[n][c], Tl, 0, 0, 0);
+                T = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf, ph[0][c], T, 0, 0, 0);
             }
 #pragma unroll
-            for (int d = 0; d < 2; d++)
-#pragma unroll
-                for (int e = 0; e < 16; e++) O[d2 + d][e] = fmaf(O[d2 + d][e], al, T[d][e]);
+            for (int e = 0; e < 16; e++) O[d][e] = fmaf(O[d][e], al, T[e] + Tl[e]);
         }
         slot ^= 1;
         store(L[slot]);
