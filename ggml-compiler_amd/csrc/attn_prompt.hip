@@ -453,13 +453,24 @@ __global__ __launch_bounds__(64 * RW * KW, RW == 1 ? 1 : 2) void k_attn_prompt(c
             }
         return;
     }
+    // The merge's maximum m is R ln 2 rounded to f32; the sums take what the rounding leaves (16 and more: 1e-6 of a
+    // split's weight, at a mask value of -65504 2e-3).
+    const float m = R * 0.693147180559945309f;
+    if (fabsf(R) < 0x1p22f) {
+        const float f = __expf(fmaf(R, -1.904654323148236017e-09f, fmaf(R, 0.693147180559945309f, -m)));  // ln 2 in two parts
+        l *= f;
+#pragma unroll
+        for (int t = 0; t < D / 32; t++)
+#pragma unroll
+            for (int e = 0; e < 16; e++) O[t][e] *= f;
+    }
     float * o = a.part_o + (sh * a.nsplit + split) * D + 4 * lk;
 #pragma unroll
     for (int t = 0; t < D / 32; t++)
 #pragma unroll
         for (int i = 0; i < 4; i++)
             *reinterpret_cast<f4_t *>(o + 32 * t + 8 * i) = f4_t{O[t][4 * i], O[t][4 * i + 1], O[t][4 * i + 2], O[t][4 * i + 3]};
-    if (lk == 0) a.part_ml[sh * a.nsplit + split] = make_float2(R * 0.693147180559945309f, l);
+    if (lk == 0) a.part_ml[sh * a.nsplit + split] = make_float2(m, l);
 }
 
 // Row groups of a workgroup for `rows` rows of a KV head: 4 (128 rows), 2, or 1 with the key blocks halved.

@@ -215,3 +215,13 @@ def test_prompt_rows_precision(gops, orc, H, Hkv, D, Sq, n_kv):
         q, kc, vc, m16 = _case(orc, H, Hkv, Sq, n_kv, D, n_kv, seed=seed)
         e += _error2(gops, q, kc, vc, m16, n_kv, D ** -0.5)
     assert np.sqrt(e[0] / e[1]) < 1.05
+
+
+@pytest.mark.parametrize("H,Hkv,D,Sq,n_kv", [(8, 8, 128, 5, 700), (8, 2, 128, 33, 523)])
+def test_prompt_rows_precision_large_scores(gops, orc, H, Hkv, D, Sq, n_kv):
+    """The same for scores of up to 13 over several splits, whose maxima are no powers of two."""
+    e = np.zeros(2)
+    for seed in (60, 70, 80, 90):
+        q, kc, vc, m16 = _case(orc, H, Hkv, Sq, n_kv, D, n_kv, seed=seed)
+        e += _error2(gops, q, kc, vc, m16, n_kv, 0.3)
+    assert np.sqrt(e[0] / e[1]) < 1.05
