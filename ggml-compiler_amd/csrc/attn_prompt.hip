@@ -13,7 +13,9 @@
 // The softmax runs in powers of two against an integer reference R >= the running maximum: raising
 // R rescales by an exact power of two and is rare, and splits with the same R merge without rounding.
 // Blocks that no row of the workgroup sees (mask all -inf: k_attn_mask_bits looks the mask over first; or
-// past the causal edge) are left out, and a block without a mask value takes no mask work.
+// past the causal edge) are left out, and a block without a mask value takes no mask work. A finite mask value
+// is added to the scaled score before the exponent, as in attn.hip: divided by the scale and added to the dot it was
+// rounded at its own size times 1 / scale (1.2 to 1.6 times the error, masks of N(0, 2), 1000 and -65504).
 //
 // Wavefronts: RW row groups x KW key halves of each block (KW = 2 where the rows are few; the halves
 // meet in LDS at the end). Grid (row tile, KV head, key split); the splits' partials have k_attn_split's
@@ -56,7 +58,7 @@ struct PromptArgs {
     int64_t m_s;
     const uint2 * bits;  // k_attn_mask_bits
     float scale2;   // |scale| * log2(e); negate: the scale is negative (Q's sign turns)
-    float mask_m;   // 1 / |scale|: a masked key's S becomes S + mask value * mask_m, as it is where the value is 0
+    float mag;      // |scale|
     bool negate;
     int Sq, H, G, n_kv, pos0, blocks, nsplit;  // blocks: key blocks per split
     float * out, * part_o;
@@ -232,52 +234,72 @@ __global__ __launch_bounds__(64 * RW * KW, RW == 1 ? 1 : 2) void k_attn_prompt(c
     while (b < b1) {
         const Lds & lds = L[slot];
         const int bn = next(b + 1);
-        load(min(bn, b1 - 1));
         // some row of this wavefront does not see every key of the block, or with a mask value
         bool some = b * KB + KB > a.n_kv;
         if constexpr (MODE == kCausal) some = some || b * KB + KB - 1 > a.pos0 + s_first;
         if constexpr (MODE == kMask) some = some || !bits || ((uint32_t) __builtin_amdgcn_readfirstlane((int) bits[b >> 5].y) >> (b & 31) & 1);
+        const int left = a.n_kv - b * KB;
+        // The block's mask values of this lane's keys k0 .. k0 + 3 (past the row's end: the last four, shifted below),
+        // loaded before the next block's K / V: a load waits for all before it.
+        const auto k0 = [&](int t, int i) { return 32 * (KW == 2 ? kw : t) + 8 * i + 4 * lk; };
+        uint64_t mw[MODE == kMask ? KT : 1][4];
+        if (MODE == kMask && some) {
+            const uint16_t * mr = a.mask + (int64_t) s * a.m_s + b * KB;
+#pragma unroll
+            for (int t = 0; t < KT; t++)
+#pragma unroll
+                for (int i = 0; i < 4; i++) __builtin_memcpy(&mw[t][i], mr + min(k0(t, i), left - 4), 8);
+            asm volatile("");
+        }
+        load(min(bn, b1 - 1));
         // Dots of D values: chains of two MFMAs, added in f32. A sum inside the MFMA is cut off, not rounded, against a
         // growing accumulator (one chain of eight: 1.10 times the error of f32 dots, four chains 0.95).
         v16f S[KT];
         const _Float16 * kp = lds.k + (32 * (KW == 2 ? kw : 0) + lr) * KP + 8 * lk;
 #pragma unroll
         for (int t = 0; t < KT; t++) {
-            v16f A[4]{};
+            const auto dot = [&](int c, int n) {  // n MFMAs from dims 16 c on
+                v16f A{};
 #pragma unroll
-            for (int c = 0; c < D / 16; c++)
-                A[c % 4] = __builtin_amdgcn_mfma_f32_32x32x16_f16(*reinterpret_cast<const h8_t *>(kp + 32 * t * KP + 16 * c), qf[c], A[c % 4], 0, 0, 0);
-            S[t] = (A[0] + A[1]) + (A[2] + A[3]);
+                for (int e = 0; e < n; e++)
+                    A = __builtin_amdgcn_mfma_f32_32x32x16_f16(*reinterpret_cast<const h8_t *>(kp + 32 * t * KP + 16 * (c + e)), qf[c + e], A, 0, 0, 0);
+                return A;
+            };
+            constexpr int n = D / 64;
+            S[t] = dot(0, n) + dot(n, n);
+            __builtin_amdgcn_sched_barrier(0);  // (all four chains at once: their registers spill others)
+            S[t] += dot(2 * n, n) + dot(3 * n, n);
         }
         float c2 = a.scale2;  // a key's exponent is c2 S
         float mx = -INFINITY;
         if (some) {
             asm volatile("");  // a branch: as selects this runs for every block
-            const uint16_t * mr = MODE == kMask ? a.mask + (int64_t) s * a.m_s : nullptr;
-            const int left = a.n_kv - b * KB, seen = MODE == kCausal ? min(left, a.pos0 + s + 1 - b * KB) : left;
+            const int seen = MODE == kCausal ? min(left, a.pos0 + s + 1 - b * KB) : left;
+            const auto value = [&](int t, int i, int r) {
+                return h2f((uint16_t) (mw[t][i] >> (16 * min(k0(t, i) - min(k0(t, i), left - 4), 3)) >> (16 * r)));
+            };
+            bool add = false;  // a mask value that is neither 0 nor -inf
 #pragma unroll
             for (int t = 0; t < KT; t++)
 #pragma unroll
-                for (int i = 0; i < 4; i++) {
-                    const int k0 = 32 * (KW == 2 ? kw : t) + 8 * i + 4 * lk;  // keys k0 .. k0 + 3 of the block
-                    uint64_t m = 0;
-                    if constexpr (MODE == kMask) {  // at the row's end, the last four values, shifted
-                        const int at = min(k0, left - 4);
-                        __builtin_memcpy(&m, mr + (b * KB + at), 8);
-                        m >>= 16 * min(k0 - at, 3);
+                for (int e = 0; e < 16; e++) {
+                    bool drop = k0(t, e >> 2) + (e & 3) >= seen;
+                    if constexpr (MODE == kMask) {
+                        const float mv = value(t, e >> 2, e & 3);
+                        drop = drop || mv == -INFINITY;
+                        add = add || (!drop && mv != 0.0f);
                     }
+                    S[t][e] = drop ? -INFINITY : S[t][e];
+                }
+            if constexpr (MODE == kMask)
+                if (__any(add)) {  // scores and values summed at the values' own size
+                    asm volatile("");
 #pragma unroll
-                    for (int r = 0; r < 4; r++) {
-                        const int e = 4 * i + r;
-                        bool drop = k0 + r >= seen;
-                        if constexpr (MODE == kMask) {
-                            const float mv = h2f((uint16_t) (m >> (16 * r)));
-                            drop = drop || mv == -INFINITY;
-                            S[t][e] = fmaf(mv, a.mask_m, S[t][e]);
-                        }
-                        S[t][e] = drop ? -INFINITY : S[t][e];
-                    }
-                    __builtin_amdgcn_sched_barrier(0);
+                    for (int t = 0; t < KT; t++)
+#pragma unroll
+                        for (int e = 0; e < 16; e++)
+                            S[t][e] = S[t][e] == -INFINITY ? S[t][e] : fmaf(S[t][e], a.mag, value(t, e >> 2, e & 3));
+                    c2 = 1.44269504088896341f;
                 }
         }
 #pragma unroll
@@ -394,9 +416,10 @@ __global__ __launch_bounds__(64 * RW * KW, RW == 1 ? 1 : 2) void k_attn_prompt(c
                 if constexpr (MODE == kMask) {
                     const float mv = h2f(a.mask[(int64_t) s * a.m_s + j]);
                     drop = drop || mv == -INFINITY;
-                    x = fmaf(mv, a.mask_m, x);
+                    x = fmaf(x, a.mag, mv) * 1.44269504088896341f;
+                } else {
+                    x *= a.scale2;
                 }
-                x *= a.scale2;
                 const float p = __builtin_amdgcn_exp2f(x - R) * kPScale;
                 if (drop || R == -INFINITY) continue;
                 const uint16_t * vj = vb + (int64_t) j * a.v_j + 4 * lk;
@@ -536,7 +559,7 @@ void launch_attn_prompt(const float * q, int64_t q_h, int64_t q_s, const void * 
     a.mask = (const uint16_t *) mask, a.m_s = m_s;
     a.scale2 = (float) (fabs((double) scale) * 1.4426950408889634074);
     a.negate = scale < 0.0f;
-    a.mask_m = (float) (1.0 / fabs((double) scale));
+    a.mag = fabsf(scale);
     a.Sq = Sq, a.H = H, a.G = H / Hkv, a.n_kv = n_kv, a.pos0 = pos0, a.blocks = p.chunk / KB, a.nsplit = p.nsplit;
     a.out = out, a.part_o = part_o, a.part_ml = part_ml;
     const int mode = mask ? kMask : pos0 >= 0 ? kCausal : kAllKeys;

@@ -225,3 +225,25 @@ def test_prompt_rows_precision_large_scores(gops, orc, H, Hkv, D, Sq, n_kv):
         q, kc, vc, m16 = _case(orc, H, Hkv, Sq, n_kv, D, n_kv, seed=seed)
         e += _error2(gops, q, kc, vc, m16, n_kv, 0.3)
     assert np.sqrt(e[0] / e[1]) < 1.05
+
+
+@pytest.mark.parametrize("H,Hkv,D,Sq,n_kv", [(8, 8, 128, 5, 700), (8, 2, 128, 33, 523), (14, 2, 64, 129, 257), (8, 2, 128, 30, 90)])
+@pytest.mark.parametrize("what", ["added", "distance", "lowest", "thousand"])
+def test_prompt_rows_precision_mask_values(gops, orc, H, Hkv, D, Sq, n_kv, what):
+    """The same for finite mask values: N(0, 2), a distance penalty, the type's lowest value on every key of half of the rows
+    (their weights come from scores rounded at 65504 in both kernels), and 1000."""
+    e = np.zeros(2)
+    for seed in (60, 70, 80, 90):
+        q, kc, vc, m16 = _case(orc, H, Hkv, Sq, n_kv, D, n_kv, seed=seed)
+        m = m16.view(np.float16).astype(np.float32)
+        if what == "added":
+            m += 2 * orc.normal((Sq, n_kv), seed=seed + 5)
+        elif what == "distance":
+            m -= np.abs(np.arange(n_kv)[None] - (n_kv - Sq + np.arange(Sq)[:, None])) / 32
+        elif what == "lowest":
+            m[::2] = -65504
+        else:
+            m += 1000
+        m16 = orc.fp32_to_fp16(m)
+        e += _error2(gops, q, kc, vc, m16, n_kv, D ** -0.5)
+    assert np.sqrt(e[0] / e[1]) < 1.05
