@@ -512,7 +512,7 @@ void run(const PromptArgs & a, int Hkv, int mode, hipStream_t s) {
 // (A mask needs rows of at least four values: launch_attn_prompt.) The scale's range: a dropped key's weight is
 // 2^(scale -inf), not 0 where the scale is 0, and a mask value is divided by the scale; k_attn_split takes the rest.
 bool attn_prompt_fits(int D, int Sq, int H, int Hkv, float scale) {
-    return (D == 64 || D == 128) && Sq > 1 && H % Hkv == 0 && (int64_t) Sq * (H / Hkv) < INT32_MAX &&
+    return (D == 64 || D == 128) && Sq > 1 && H % Hkv == 0 && H / Hkv <= 8 && (int64_t) Sq * (H / Hkv) < INT32_MAX &&
            fabsf(scale) >= 0x1p-60f && fabsf(scale) <= 0x1p60f;
 }
 
@@ -543,7 +543,7 @@ void launch_attn_prompt(const float * q, int64_t q_h, int64_t q_s, const void * 
                         const void * v, int64_t v_h, int64_t v_j, const void * mask, int64_t m_s, int pos0, int D, int Sq,
                         int H, int Hkv, int n_kv, float scale, float * out, float * part_o, float2 * part_ml,
                         const AttnPlan & p, void * bits, hipStream_t s) {
-    require(attn_prompt_fits(D, Sq, H, Hkv, scale), "attn prompt: D 64 or 128, more than one query row, a scale within 2^-60 .. 2^60");
+    require(attn_prompt_fits(D, Sq, H, Hkv, scale), "attn prompt: D 64 or 128, several query rows, at most 8 heads per KV head, a scale within 2^-60 .. 2^60");
     require(p.chunk % KB == 0 && (int64_t) p.nsplit * p.chunk >= n_kv, "attn prompt: the splits must cover the keys");
     require(((int64_t) Sq * (H / Hkv) / 32 + 1) * Hkv * p.nsplit < INT32_MAX, "attn prompt: too many row tiles");
     require(!out || p.nsplit == 1, "attn prompt: several splits go to the merge");

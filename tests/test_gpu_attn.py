@@ -247,3 +247,13 @@ def test_prompt_rows_precision_mask_values(gops, orc, H, Hkv, D, Sq, n_kv, what)
         m16 = orc.fp32_to_fp16(m)
         e += _error2(gops, q, kc, vc, m16, n_kv, D ** -0.5)
     assert np.sqrt(e[0] / e[1]) < 1.05
+
+
+@pytest.mark.parametrize("D", [64, 128, 256])
+@pytest.mark.parametrize("Sq", [1, 2, 40])
+def test_more_than_8_heads_per_kv_head_refused(gops, orc, D, Sq):
+    """The C API's bound (include/gcq.h), for one query row and several, with and without a mask."""
+    q, kc, vc, m16 = _case(orc, 9, 1, Sq, 70, D, 70, seed=54)
+    for m in (m16, None):
+        with pytest.raises(Exception, match="8 query heads"):
+            _run(gops, q, kc, vc, m, 70, 0.1)
