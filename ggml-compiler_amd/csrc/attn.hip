@@ -755,6 +755,18 @@ static void launch_merge(int D, const float * po, const float2 * pml, float * ou
     check_launch("flash_attn merge");
 }
 
+// Calls of several query rows that k_attn_split answers sooner than k_attn_prompt (over one block of 64 keys, which needs
+// no merge there). Kernel times on 8 KV heads of 128, per-row / matrix cores: two or three rows of a KV head fill
+// 1/16 of a row tile, so the keys' reads alone count: 2 rows over 1000 keys 9.7 / 16.8 us, over 32768 35 / 39; up to
+// about 400 MB of K and V over all query rows, which read them again (4 rows over 32768 keys: 45 / 35). And short calls of
+// one query head per KV head (of 128: two): 16 rows over 256 keys 9.4 / 14.3, over 1000 12.5 / 15.3, but 33 rows over 1000
+// 19.9 / 14.8, and with four heads 16 rows over 256 keys 15.6 / 15.3.
+static bool attn_few_rows(int D, int Sq, int H, int Hkv, int n_kv) {
+    const int64_t rows = (int64_t) Sq * (H / Hkv), keys = (int64_t) Hkv * n_kv;
+    if (n_kv <= 64) return false;
+    return (rows <= 4 && Sq * keys * D * 4 <= 400000000) || (H / Hkv <= (D == 128 ? 2 : 1) && rows * keys <= 131072);
+}
+
 void launch_flash_attn(const float * q, int64_t q_h, int64_t q_s, const void * k, int64_t k_h, int64_t k_j,
                        const void * v, int64_t v_h, int64_t v_j, const void * mask, int64_t m_s, float * out, int D,
                        int Dv, int Sq, int H, int Hkv, int n_kv, float scale, void * ws, size_t ws_size,
@@ -780,7 +792,8 @@ void launch_flash_attn(const float * q, int64_t q_h, int64_t q_s, const void * k
         check_launch("flash_attn merge");
         return;
     }
-    if (attn_prompt_fits(D, Sq, H, Hkv, scale) && (!mask || n_kv >= 4) && k_j < (1 << 24) && v_j < (1 << 24)) {
+    if (attn_prompt_fits(D, Sq, H, Hkv, scale) && !attn_few_rows(D, Sq, H, Hkv, n_kv) && (!mask || n_kv >= 4) &&
+        k_j < (1 << 24) && v_j < (1 << 24)) {
         const AttnPlan pp = attn_plan_prompt(Sq, H, Hkv, n_kv);
         const size_t bits = attn_prompt_bits(Sq, H, Hkv, n_kv);  // the workspace: bits, then the partials
         po = (float *) ((uint8_t *) ws + bits);

@@ -114,13 +114,12 @@ __global__ __launch_bounds__(1024) void k_attn_mask_bits(const uint16_t * __rest
     if (tid == 0) bits[(int64_t) blockIdx.y * gridDim.x + blockIdx.x] = make_uint2(sh[0], sh[1]);
 }
 
-template <int D, int RW, int KW, int MODE>
+template <int D, int RW, int KW, int NP, int MODE>
 __global__ __launch_bounds__(64 * RW * KW, RW == 1 ? 1 : 2) void k_attn_prompt(const PromptArgs a) {
     constexpr int NW = RW * KW, NT = 64 * NW, KT = 2 / KW;
     constexpr int KP = D + 8;                       // pitch of a K row (halves)
     constexpr int KL = KB * (D / 8) / NT;           // 16-byte K pieces per thread
     constexpr int VL = (D / 32) * (KB / 32) / NW;   // 4-key x 4-dim V tiles per lane
-    constexpr int NP = RW <= 2 ? 3 : 2;             // f16 parts of a weight
     struct Lds {
         _Float16 k[KB * KP];
         _Float16 v[D * VP];
@@ -225,7 +224,22 @@ __global__ __launch_bounds__(64 * RW * KW, RW == 1 ? 1 : 2) void k_attn_prompt(c
         for (int e = 0; e < 16; e++) O[t][e] = 0.0f;
     float R = -INFINITY, l = 0.0f;  // reference exponent (an integer) and this lane's half of the weights' sum
 
+    // A block's mask values of this lane's keys k0 .. k0 + 3 (past the row's end: the last four, shifted where they are
+    // used). KW == 1 loads them at the block's start, before the next block's K and V (a load waits for all before it); KW == 2,
+    // whose rows are few and whose registers are not, a block ahead.
+    const auto k0 = [&](int t, int i) { return 32 * (KW == 2 ? kw : t) + 8 * i + 4 * lk; };
+    uint64_t mw[MODE == kMask ? KT : 1][4];
+    const auto load_mask = [&](int b) {
+        const uint16_t * mr = a.mask + (int64_t) s * a.m_s + b * KB;
+#pragma unroll
+        for (int t = 0; t < (MODE == kMask ? KT : 1); t++)
+#pragma unroll
+            for (int i = 0; i < 4; i++) __builtin_memcpy(&mw[t][i], mr + min(k0(t, i), a.n_kv - b * KB - 4), 8);
+        asm volatile("");
+    };
+
     int b = next(b0), slot = 0;
+    if (MODE == kMask && KW == 2 && b < b1) load_mask(b);
     if (b < b1) {
         load(b);
         store(L[0]);
@@ -239,18 +253,7 @@ __global__ __launch_bounds__(64 * RW * KW, RW == 1 ? 1 : 2) void k_attn_prompt(c
         if constexpr (MODE == kCausal) some = some || b * KB + KB - 1 > a.pos0 + s_first;
         if constexpr (MODE == kMask) some = some || !bits || ((uint32_t) __builtin_amdgcn_readfirstlane((int) bits[b >> 5].y) >> (b & 31) & 1);
         const int left = a.n_kv - b * KB;
-        // The block's mask values of this lane's keys k0 .. k0 + 3 (past the row's end: the last four, shifted below),
-        // loaded before the next block's K / V: a load waits for all before it.
-        const auto k0 = [&](int t, int i) { return 32 * (KW == 2 ? kw : t) + 8 * i + 4 * lk; };
-        uint64_t mw[MODE == kMask ? KT : 1][4];
-        if (MODE == kMask && some) {
-            const uint16_t * mr = a.mask + (int64_t) s * a.m_s + b * KB;
-#pragma unroll
-            for (int t = 0; t < KT; t++)
-#pragma unroll
-                for (int i = 0; i < 4; i++) __builtin_memcpy(&mw[t][i], mr + min(k0(t, i), left - 4), 8);
-            asm volatile("");
-        }
+        if (MODE == kMask && KW == 1 && some) load_mask(b);
         load(min(bn, b1 - 1));
         // Dots of D values: chains of two MFMAs, added in f32. A sum inside the MFMA is cut off, not rounded, against a
         // growing accumulator (one chain of eight: 1.10 times the error of f32 dots, four chains 0.95).
@@ -258,17 +261,18 @@ __global__ __launch_bounds__(64 * RW * KW, RW == 1 ? 1 : 2) void k_attn_prompt(c
         const _Float16 * kp = lds.k + (32 * (KW == 2 ? kw : 0) + lr) * KP + 8 * lk;
 #pragma unroll
         for (int t = 0; t < KT; t++) {
-            const auto dot = [&](int c, int n) {  // n MFMAs from dims 16 c on
+            const auto dot = [&](int c) {  // dims 16 c .. 16 c + 31
                 v16f A{};
 #pragma unroll
-                for (int e = 0; e < n; e++)
+                for (int e = 0; e < 2; e++)
                     A = __builtin_amdgcn_mfma_f32_32x32x16_f16(*reinterpret_cast<const h8_t *>(kp + 32 * t * KP + 16 * (c + e)), qf[c + e], A, 0, 0, 0);
                 return A;
             };
-            constexpr int n = D / 64;
-            S[t] = dot(0, n) + dot(n, n);
-            __builtin_amdgcn_sched_barrier(0);  // (all four chains at once: their registers spill others)
-            S[t] += dot(2 * n, n) + dot(3 * n, n);
+            S[t] = dot(0) + dot(2);
+            if constexpr (D == 128) {
+                __builtin_amdgcn_sched_barrier(0);  // (all four chains at once: their registers spill others)
+                S[t] += dot(4) + dot(6);
+            }
         }
         float c2 = a.scale2;  // a key's exponent is c2 S
         float mx = -INFINITY;
@@ -302,6 +306,7 @@ __global__ __launch_bounds__(64 * RW * KW, RW == 1 ? 1 : 2) void k_attn_prompt(c
                     c2 = 1.44269504088896341f;
                 }
         }
+        if (MODE == kMask && KW == 2) load_mask(min(bn, b1 - 1));
 #pragma unroll
         for (int t = 0; t < KT; t++)
 #pragma unroll
@@ -499,12 +504,26 @@ __global__ __launch_bounds__(64 * RW * KW, RW == 1 ? 1 : 2) void k_attn_prompt(c
 // Row groups of a workgroup for `rows` rows of a KV head: 4 (128 rows), 2, or 1 with the key blocks halved.
 int row_groups(int64_t rows) { return rows <= 32 ? 1 : rows <= 64 ? 2 : 4; }
 
-template <int D, int RW, int KW>
+template <int D, int RW, int KW, int NP>
 void run(const PromptArgs & a, int Hkv, int mode, hipStream_t s) {
     const unsigned grid = (unsigned) (((int64_t) a.Sq * a.G + 32 * RW - 1) / (32 * RW) * Hkv * a.nsplit);
-    if (mode == kMask) k_attn_prompt<D, RW, KW, kMask><<<grid, 64 * RW * KW, 0, s>>>(a);
-    else if (mode == kCausal) k_attn_prompt<D, RW, KW, kCausal><<<grid, 64 * RW * KW, 0, s>>>(a);
-    else k_attn_prompt<D, RW, KW, kAllKeys><<<grid, 64 * RW * KW, 0, s>>>(a);
+    if (mode == kMask) k_attn_prompt<D, RW, KW, NP, kMask><<<grid, 64 * RW * KW, 0, s>>>(a);
+    else if (mode == kCausal) k_attn_prompt<D, RW, KW, NP, kCausal><<<grid, 64 * RW * KW, 0, s>>>(a);
+    else k_attn_prompt<D, RW, KW, NP, kAllKeys><<<grid, 64 * RW * KW, 0, s>>>(a);
+}
+
+// Weights in three parts where the keys are few enough for single weights to show (up to 64 rows and 512 keys: 3 rows over 4
+// keys 1.0 of the per-row kernel's error, 1.07 in two parts); two beyond (6 rows over 32768 keys, 32 heads of 64: 81 us in
+// three, 68 in two) and for more rows, where the third costs most (512 rows over 4096 keys: 136 us and 92).
+constexpr int kFewKeys = 512;
+template <int D>
+void run_rows(const PromptArgs & a, int Hkv, int mode, int rg, hipStream_t s) {
+    const bool few = a.n_kv <= kFewKeys;
+    if (rg == 4) run<D, 4, 1, 2>(a, Hkv, mode, s);
+    else if (rg == 2 && few) run<D, 2, 2, 3>(a, Hkv, mode, s);
+    else if (rg == 2) run<D, 2, 2, 2>(a, Hkv, mode, s);
+    else if (few) run<D, 1, 2, 3>(a, Hkv, mode, s);
+    else run<D, 1, 2, 2>(a, Hkv, mode, s);
 }
 
 }  // namespace
@@ -516,13 +535,14 @@ bool attn_prompt_fits(int D, int Sq, int H, int Hkv, float scale) {
            fabsf(scale) >= 0x1p-60f && fabsf(scale) <= 0x1p60f;
 }
 
-// Key splits: about 512 workgroups in all (two per CU), each split of at least two key blocks (no more for a
-// smaller n_kv, so a bound for every KV length up to n_kv).
+// Key splits: about 512 workgroups in all (two per CU), each split of at least two key blocks, or one where that makes
+// few splits to merge (8; 16 for up to 256 output rows): 33 rows over 300 keys 23.0 us in two splits of three blocks, 16.1 in
+// five of one. No more for a smaller n_kv, so a bound for every KV length up to n_kv.
 int attn_prompt_max_split(int Sq, int H, int Hkv, int n_kv) {
     const int64_t rows = (int64_t) Sq * (H / Hkv), tile = 32 * row_groups(rows);
     const int64_t wgs = (rows + tile - 1) / tile * Hkv;
     const int nblk = (n_kv + KB - 1) / KB;
-    return (int) std::max<int64_t>(1, std::min<int64_t>({512 / wgs, nblk / 2, 64}));
+    return (int) std::max<int64_t>(1, std::min<int64_t>({512 / wgs, std::max(std::min(nblk, (int64_t) Sq * H <= 256 ? 16 : 8), nblk / 2), 64}));
 }
 AttnPlan attn_plan_prompt(int Sq, int H, int Hkv, int n_kv) {
     const int nblk = (n_kv + KB - 1) / KB, most = attn_prompt_max_split(Sq, H, Hkv, n_kv);
@@ -564,7 +584,7 @@ void launch_attn_prompt(const float * q, int64_t q_h, int64_t q_s, const void * 
     a.out = out, a.part_o = part_o, a.part_ml = part_ml;
     const int mode = mask ? kMask : pos0 >= 0 ? kCausal : kAllKeys;
     const int rg = row_groups((int64_t) Sq * a.G);
-    if (mask && n_kv > kBitsKeys) {
+    if (mask && n_kv > kBitsKeys && rg == 4) {
         const int tile = 32 * rg;
         const int64_t tiles = ((int64_t) Sq * a.G + tile - 1) / tile;
         require(bits && tiles <= 65535, "attn prompt: a mask needs its bits' workspace and at most 65535 row tiles");
@@ -572,15 +592,8 @@ void launch_attn_prompt(const float * q, int64_t q_h, int64_t q_s, const void * 
         k_attn_mask_bits<<<dim3((unsigned) ((n_kv + 32 * KB - 1) / (32 * KB)), (unsigned) tiles), 1024, 0, s>>>(
             a.mask, m_s, Sq, a.G, n_kv, tile, (uint2 *) bits);
     }
-    if (D == 64) {
-        if (rg == 1) run<64, 1, 2>(a, Hkv, mode, s);
-        else if (rg == 2) run<64, 2, 2>(a, Hkv, mode, s);
-        else run<64, 4, 1>(a, Hkv, mode, s);
-    } else {
-        if (rg == 1) run<128, 1, 2>(a, Hkv, mode, s);
-        else if (rg == 2) run<128, 2, 2>(a, Hkv, mode, s);
-        else run<128, 4, 1>(a, Hkv, mode, s);
-    }
+    if (D == 64) run_rows<64>(a, Hkv, mode, rg, s);
+    else run_rows<128>(a, Hkv, mode, rg, s);
     check_launch("attn prompt");
 }
 
