@@ -217,7 +217,7 @@ def test_prompt_rows_precision(gops, orc, H, Hkv, D, Sq, n_kv):
     assert np.sqrt(e[0] / e[1]) < 1.05
 
 
-@pytest.mark.parametrize("H,Hkv,D,Sq,n_kv", [(8, 8, 128, 5, 700), (8, 2, 128, 33, 523)])
+@pytest.mark.parametrize("H,Hkv,D,Sq,n_kv", [(8, 2, 128, 5, 700), (8, 2, 128, 33, 523)])
 def test_prompt_rows_precision_large_scores(gops, orc, H, Hkv, D, Sq, n_kv):
     """The same for scores of up to 13 over several splits, whose maxima are no powers of two."""
     e = np.zeros(2)
@@ -227,7 +227,7 @@ def test_prompt_rows_precision_large_scores(gops, orc, H, Hkv, D, Sq, n_kv):
     assert np.sqrt(e[0] / e[1]) < 1.05
 
 
-@pytest.mark.parametrize("H,Hkv,D,Sq,n_kv", [(8, 8, 128, 5, 700), (8, 2, 128, 33, 523), (14, 2, 64, 129, 257), (8, 2, 128, 30, 90)])
+@pytest.mark.parametrize("H,Hkv,D,Sq,n_kv", [(8, 2, 128, 5, 700), (8, 2, 128, 33, 523), (14, 2, 64, 129, 257), (8, 2, 128, 30, 90)])
 @pytest.mark.parametrize("what", ["added", "distance", "lowest", "thousand"])
 def test_prompt_rows_precision_mask_values(gops, orc, H, Hkv, D, Sq, n_kv, what):
     """The same for finite mask values: N(0, 2), a distance penalty, the type's lowest value on every key of half of the rows
