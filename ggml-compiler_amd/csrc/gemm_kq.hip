@@ -441,15 +441,19 @@ void run_kq(const void * wv, int64_t N, int64_t K, const void * act, int64_t M, 
     a.ldy = (int) ldy;
     a.raw_sb = raw_sb;
     const auto tiles = [&](int64_t tm, int64_t tn) { return ((M + tm - 1) / tm) * ((N + tn - 1) / tn); };
-    // 64 x 128 tiles when there are more of them than CUs; else 64 x 64 in two K groups; when even those
-    // cover less than half the CUs, 32 x 32 in eight (512 x 4096 x 14336: 94 us in 512 tiles of 64 x 64,
-    // 114 in 256 of 64 x 128 without groups; 128 x 4096 x 4096: 17 us in 512 tiles of 32 x 32, 24 in 128
-    // of 64 x 64 without groups)
+    // 64 x 128 tiles where they fill the chip; else 64 x 64 in two K groups; where 32 x 32 tiles are few, those in
+    // eight. Each K group needs super-blocks: one, and groups only wait; two, and eight groups do the work of two;
+    // below eight, 64 x 128 tiles are worth half as many of them and 32 x 32 tiles only one per CU. Kernel times, Q4_K, us for
+    // 64 x 128 / 64 x 64 / 32 x 32 tiles: 512 x 4096 x 14336 115 / 92 / 164; 128 x 4096 x 4096 32 / 21 / 19; 128 x 4096 x 256
+    // 6.2 / 7.1 / 11.2; 256 x 2048 x 512 8.2 / 7.3 / 11.7; 65 x 4096 x 1024 11.3 / 8.9 / 11.3; 33 x 4096 x 1024 10.9 / 8.3 / 6.9.
+    // 765 shapes of 9 to 2048 rows, 96 to 128256 columns and K 256 to 14336: within 1 % of the best of the three on average
+    // for each type, at most 17 % off it.
     if constexpr (RAW) {
         k_gemm_kq<TYPE, 2, 4, 1, RAW><<<(unsigned) tiles(64, 128), 256, 0, s>>>(a);
     } else {
-        if (tiles(64, 128) > cu_count()) k_gemm_kq<TYPE, 2, 4, 1, RAW><<<(unsigned) tiles(64, 128), 256, 0, s>>>(a);
-        else if (tiles(64, 64) > cu_count() / 2) k_gemm_kq<TYPE, 2, 2, 2, RAW><<<(unsigned) tiles(64, 64), 256, 0, s>>>(a);
+        const int64_t cus = cu_count();
+        if (a.nsb == 1 || tiles(64, 128) > (a.nsb < 8 ? cus / 2 : cus)) k_gemm_kq<TYPE, 2, 4, 1, RAW><<<(unsigned) tiles(64, 128), 256, 0, s>>>(a);
+        else if (a.nsb == 2 || tiles(32, 32) > (a.nsb < 8 ? cus : 2 * cus)) k_gemm_kq<TYPE, 2, 2, 2, RAW><<<(unsigned) tiles(64, 64), 256, 0, s>>>(a);
         else k_gemm_kq<TYPE, 1, 1, 8, RAW><<<(unsigned) tiles(32, 32), 512, 0, s>>>(a);
     }
 }

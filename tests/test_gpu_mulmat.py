@@ -312,10 +312,11 @@ def test_gemm_kquant_prefill_shape_row_slices(gops, orc, t, N, K):
 
 
 @pytest.mark.parametrize("t", KQ)
-@pytest.mark.parametrize("M,N,K", [(9, 31, 256), (33, 65, 2304), (64, 8200, 768), (65, 8193, 512), (70, 16500, 256)])
+@pytest.mark.parametrize("M,N,K", [(9, 31, 256), (33, 65, 2304), (64, 8200, 768), (65, 8193, 512), (70, 16500, 256),
+                                   (40, 300, 768), (33, 900, 512)])
 def test_gemm_kquant_k_groups(gops, orc, t, M, N, K):
-    """Each tile of the K-quant GEMM at its edges: 32 x 32 tiles in eight K groups (one super-block: seven
-    groups idle; nine: a second round for one group), 64 x 64 in two (three super-blocks), 64 x 128.
+    """Each tile of the K-quant GEMM at its edges: 32 x 32 tiles in eight K groups (three super-blocks: five
+    groups idle; nine: a second round for one group), 64 x 64 in two (two and three super-blocks), 64 x 128.
     Integer sums are exact, so only f32 sums of K / 256 terms differ: 1e-5 covers any order of them."""
     raw, qw = _weight(gops, orc, t, N, K, 41)
     x = orc.normal((M, K), seed=42)
