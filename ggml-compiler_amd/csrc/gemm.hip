@@ -492,14 +492,23 @@ static void run_gemm(const void * wv, int64_t N, int64_t K, const void * act, in
     const int nb = (int) (K / 32), m = (int) M, n = (int) N, ld = (int) ldy;
     const auto tiles = [&](int64_t tm, int64_t tn) { return ((M + tm - 1) / tm) * ((N + tn - 1) / tn); };
     const int64_t cus = cu_count(), t32 = tiles(32, 32), t128 = tiles(128, 128);
-    // A 32 x 32 tile costs about 20 us per 4 CUs' worth of tiles at K = 4096 whatever their number; 128 x 128
-    // tiles in two K groups cost 53-65 us up to a tile per CU (each workgroup's serial chain over K), without
-    // groups 72. Where they meet: 500 x 4096 (8 tiles of 32 per CU) 43 / 55 us, 500 x 6144 (12) 62 / 60,
-    // 500 x 8192 (16) 81 / 65. More than one 128 x 128 tile per CU: two workgroups share it and groups only add the
-    // sums (512 x 14336: 97 us, 118 in two groups). Eight wavefronts per 32 x 32 tile for up to 1.5 tiles per
-    // CU (33 x 4096 x 14336: 23 us, 31 in four), four for more (33 x 14336 x 4096: 26 / 24).
+    // Kernel times at K = 4096, us, for 32 x 32 tiles in eight and in four wavefronts and 128 x 128 tiles in two K groups
+    // and without. 32 x 32 tiles: about 9 us plus 5 for every tile per CU; 128 x 128 tiles in two groups 50-70 up to a
+    // tile per CU (each workgroup's serial chain over K). They meet at 11 32 x 32 tiles per CU. With more than one
+    // 128 x 128 tile per CU two workgroups share it and groups only add the sums. Up to 32 rows fill a quarter of a 128-row tile
+    // at most, whatever N is.
+    //                      Q4_0                       Q8_0
+    //   33 x 4096       9.5 / 12.8 / 50 / 69      11 /  13 /  53 /  67
+    //   512 x 2048       27 /  26 /  59 / 72      33 /  28 /  59 /  70
+    //   512 x 4096       49 /  45 /  60 / 74      63 /  48 /  63 /  72
+    //   1024 x 4096     104 /  94 /  68 / 81     135 /  98 /  71 /  79
+    //   129 x 32000     108 / 102 / 123 / 99     140 / 102 / 125 / 100
+    //   16 x 128256     100 /  96 / 218 / 210    144 / 130 / 248 / 194
+    //   32 x 128256     123 / 117 / 232 / 214    175 / 151 / 259 / 234
+    // 765 shapes of 9 to 2048 rows, 96 to 128256 columns and K 256 to 14336: within 1 % of the best of the four on average for
+    // both types; the farthest off it 39 % (Q8_0 129 x 2048 x 256) and 30 % (Q8_0 33 x 128256 x 4096).
     if (2 * t32 <= 3 * cus) k_gemm_kg<TYPE, 4, 8><<<(unsigned) t32, 512, 0, s>>>(qs, d, xc, xm, y, res, m, n, nb, ld);
-    else if (t32 <= 11 * cus) k_gemm_kg<TYPE, 4, 4><<<(unsigned) t32, 256, 0, s>>>(qs, d, xc, xm, y, res, m, n, nb, ld);
+    else if (t32 <= 11 * cus || m <= 32) k_gemm_kg<TYPE, 4, 4><<<(unsigned) t32, 256, 0, s>>>(qs, d, xc, xm, y, res, m, n, nb, ld);
     else if (t128 <= cus) k_gemm<TYPE, false, 2><<<(unsigned) t128, 512, 0, s>>>(qs, d, xc, xm, y, res, nullptr, m, n, nb, ld, 0);
     else k_gemm<TYPE, false, 1><<<(unsigned) t128, 256, 0, s>>>(qs, d, xc, xm, y, res, nullptr, m, n, nb, ld, 0);
 }

@@ -326,11 +326,11 @@ def test_gemm_kquant_k_groups(gops, orc, t, M, N, K):
 
 @pytest.mark.parametrize("t", ["q4_0", "q8_0"])
 @pytest.mark.parametrize("M,N,K", [(9, 31, 32), (33, 65, 96), (40, 200, 1056), (33, 6200, 160), (97, 16300, 288),
-                                   (300, 9100, 160), (129, 24800, 96)])
+                                   (300, 9100, 160), (129, 24800, 96), (17, 90200, 96)])
 def test_gemm_k_groups(gops, orc, t, M, N, K):
     """Each tile of the GEMM at its edges: 32 x 32 tiles in eight K groups (fewer blocks than a step, a step that
-    starts early) and in four, 128 x 128 in two groups (one group a chunk short) and without, each also onto a
-    residual. Block sums are exact, so only f32 sums of K / 32 terms differ: 1e-5 covers any order of them."""
+    starts early) and in four (and for up to 32 rows of any width), 128 x 128 in two groups (one group a chunk
+    short) and without, each also onto a residual. Block sums are exact, so only f32 sums of K / 32 terms differ: 1e-5 covers any order of them."""
     raw, qw = _weight(gops, orc, t, N, K, 43)
     x = orc.normal((M, K), seed=44)
     ref = orc.mul_mat(raw, t, x, K)
