@@ -161,6 +161,51 @@ def test_prompt_rows_scales(gops, orc, D, n_kv, masked, scale):
     assert orc.parity(out, orc.flash_attn_ext(q, kc, vc, m16, scale)) < 1e-5
 
 
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("n_kv", [2048, 2049, 2111, 4160])
+@pytest.mark.parametrize("what", ["causal", "far", "border", "scattered"])
+def test_prompt_rows_mask_block_words(gops, orc, D, n_kv, what):
+    """Masks of more than 2048 keys over several row tiles: a word of the mask's block bits holds 32 blocks of 64 keys.
+    Causal masks; tiles that see nothing of the first word, or nothing at all; visible keys only on both sides of the
+    word's border; and single visible blocks far apart."""
+    H, Hkv, Sq = 8, 2, 100
+    q, kc, vc, m16 = _case(orc, H, Hkv, Sq, n_kv, D, n_kv + 3, seed=55)
+    if what != "causal":
+        m = np.full((Sq, n_kv), -np.inf, np.float32)
+        if what == "far":
+            m[:32, n_kv - 40:] = 0  # the first tile of 128 (query, head) rows; the second sees nothing
+            m[64:, :5] = 0
+        elif what == "border":
+            m[:, 2048 - 70:2048 - 60] = 0
+            m[:, 2047:2050] = 0
+        else:
+            m[np.arange(Sq), (np.arange(Sq) * 61) % n_kv] = 0
+            m[:, n_kv - 1] = 0
+        m16 = orc.fp32_to_fp16(m)
+    out = _run(gops, q, kc, vc, m16, n_kv, D ** -0.5)
+    assert orc.parity(out, orc.flash_attn_ext(q, kc[:, :n_kv], vc[:, :n_kv], m16, D ** -0.5)) < 1e-5
+
+
+@pytest.mark.parametrize("H,Hkv,D,Sq,n_kv", [(8, 2, 64, 5, 300), (8, 2, 128, 13, 700), (8, 2, 128, 70, 2200), (14, 2, 64, 3, 9000)])
+@pytest.mark.parametrize("masked", [True, False])
+def test_prompt_rows_interleaved_cache(gops, orc, H, Hkv, D, Sq, n_kv, masked):
+    """K and V rows farther apart than D ([ctx, Hkv, D + pad] caches viewed as [Hkv, ctx, D], K and V of different pads), q
+    rows in both orders; at 9000 keys more than 32 splits meet in the merge."""
+    q, kc, vc, m16 = _case(orc, H, Hkv, Sq, n_kv, D, n_kv, seed=56)
+
+    def view(c, pad):
+        t = torch.zeros((n_kv, Hkv, D + pad), dtype=torch.float16, device="cuda")
+        t[:, :, :D] = torch.from_numpy(c.view(np.float16)).cuda().transpose(0, 1)
+        return t[:, :, :D].transpose(0, 1)
+
+    tq = torch.from_numpy(q).cuda()
+    tm = torch.from_numpy(m16.view(np.float16)).cuda() if masked else None
+    ref = orc.flash_attn_ext(q, kc, vc, m16 if masked else None, 0.1)
+    for qq in (tq, tq.transpose(0, 1).contiguous().transpose(0, 1)):
+        out = to_np(gops.flash_attn_ext(qq, view(kc, 8), view(vc, 24), tm, 0.1, n_kv=n_kv))
+        assert orc.parity(out, ref) < 1e-5
+
+
 def _same_with_infinities(out, ref, tol):
     for kind in (np.isnan, np.isposinf, np.isneginf):
         assert np.array_equal(kind(out), kind(ref)), kind.__name__

@@ -342,17 +342,21 @@ def test_gemm_k_groups(gops, orc, t, M, N, K):
     assert orc.parity(y, ref + res) < 1e-5
 
 
+@pytest.mark.parametrize("t", ["q8_0", "q4_0"])
 @pytest.mark.parametrize("M,N", [(9, 64), (33, 6200), (300, 9100), (129, 24800)])
-def test_gemm_infinite_weight_scale(gops, orc, M, N):
+def test_gemm_infinite_weight_scale(gops, orc, t, M, N):
     """A block with an infinite scale gives isum * inf, not a NaN from inf - inf: the sign of its block sum."""
     K = 64
-    raw, _ = _weight(gops, orc, "q8_0", N, K, 46)
+    raw, _ = _weight(gops, orc, t, N, K, 46)
     raw = raw.copy().reshape(N, -1)
     raw[5, 0:2] = [0x00, 0x7C]  # d of row 5's first block: +inf
-    qw = gops.QuantWeight.from_ggml(torch.from_numpy(raw), "q8_0", K)
+    qw = gops.QuantWeight.from_ggml(torch.from_numpy(raw), t, K)
     x = torch.ones((M, K), device="cuda")
-    q = raw[5, 2:34].view(np.int8)
-    assert q.astype(np.int64).sum() != 0
+    if t == "q8_0":
+        total = raw[5, 2:34].view(np.int8).astype(np.int64).sum()
+    else:
+        total = (raw[5, 2:18] & 15).astype(np.int64).sum() + (raw[5, 2:18] >> 4).sum() - 8 * 32
+    assert total != 0
     y = to_np(gops.mul_mat(qw, x))
-    assert np.all(y[:, 5] == np.sign(q.astype(np.int64).sum()) * np.inf)
+    assert np.all(y[:, 5] == np.sign(total) * np.inf)
     assert np.all(np.isfinite(np.delete(y, 5, axis=1)))
