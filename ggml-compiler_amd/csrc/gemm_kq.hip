@@ -220,7 +220,7 @@ __device__ __forceinline__ h8_t bytes_to_h8(uint32_t b0, uint32_t b1) {
     return o;
 }
 
-template <int TYPE, int XT, int WN, int KG, bool RAW>
+template <int TYPE, int XT, int WN, int KG, bool RAW, class Sum = float>
 __global__ __launch_bounds__(64 * WN * KG, 2) void k_gemm_kq(const KqArgs a) {
     constexpr int TM = 32 * XT, TN = 32 * WN, NT = 64 * WN, AP = 4 * XT / WN;
     constexpr int SHIFT = TYPE == T_Q6_K ? 6 : 3;
@@ -229,7 +229,7 @@ __global__ __launch_bounds__(64 * WN * KG, 2) void k_gemm_kq(const KqArgs a) {
         KqCodes<TYPE, XT, WN> c[2];
         KqScales<TYPE, XT> s[2];
     };
-    constexpr size_t kRed = KG > 1 ? (size_t) (KG - 1) * WN * XT * 1024 * 4 : 0;  // the groups' sums
+    constexpr size_t kRed = KG > 1 ? (size_t) (KG - 1) * WN * XT * 1024 * sizeof(Sum) : 0;  // the groups' sums
     constexpr size_t kLds = sizeof(Lds) * KG > kRed ? sizeof(Lds) * KG : kRed;
     __shared__ __align__(16) uint8_t lds[kLds];
     const int mt = (a.M + TM - 1) / TM, nt = (a.N + TN - 1) / TN, total = mt * nt;
@@ -279,10 +279,8 @@ __global__ __launch_bounds__(64 * WN * KG, 2) void k_gemm_kq(const KqArgs a) {
         if constexpr (TYPE == T_Q6_K) hd.d = a.wd[bi + sb];
     };
 
-    v16f acc[XT];
+    Sum acc[XT][16]{};
     v16i ih[XT], il[XT];
-#pragma unroll
-    for (int x = 0; x < XT; x++) acc[x] = v16f{};
 
     // This group's super-blocks: the same number of rounds for every group (barriers), a round past the
     // end computing nothing. Loads past the end read the last super-block again: a load under a
@@ -376,7 +374,7 @@ __global__ __launch_bounds__(64 * WN * KG, 2) void k_gemm_kq(const KqArgs a) {
                                     const int e = 4 * q + r;
                                     float v = dw * (float) ((ih[x][e] << SHIFT) + il[x][e]);
                                     if constexpr (Kq<TYPE>::MIN) v = fmaf(-dm, i2[e], v);
-                                    acc[x][e] = fmaf(dx[r], v, acc[x][e]);
+                                    acc[x][e] = __builtin_elementwise_fma((Sum) dx[r], (Sum) v, acc[x][e]);
                                 }
                             }
                         }
@@ -389,21 +387,32 @@ __global__ __launch_bounds__(64 * WN * KG, 2) void k_gemm_kq(const KqArgs a) {
     }
     if constexpr (RAW) return;
 
-    if constexpr (KG > 1) {  // groups 1.. hand their sums to group 0, added in the groups' order
-        float * red = reinterpret_cast<float *>(lds) + (size_t) (wave % WN) * XT * 1024 + lane;
+    if constexpr (KG > 1) {  // groups 1.. hand their sums to group 0, which adds them in pairs
+        static_assert((KG & (KG - 1)) == 0, "pairs of groups");
+        constexpr int RS = WN * XT * 1024;
+        Sum * red = reinterpret_cast<Sum *>(lds) + (size_t) (wave % WN) * XT * 1024 + lane;
         if (kg > 0) {
 #pragma unroll
             for (int x = 0; x < XT; x++)
 #pragma unroll
-                for (int r = 0; r < 16; r++) red[(size_t) (kg - 1) * WN * XT * 1024 + x * 1024 + r * 64] = acc[x][r];
+                for (int r = 0; r < 16; r++) red[(size_t) (kg - 1) * RS + x * 1024 + r * 64] = acc[x][r];
         }
         __syncthreads();
         if (kg > 0) return;
-        for (int g = 0; g < KG - 1; g++)
 #pragma unroll
-            for (int x = 0; x < XT; x++)
+        for (int x = 0; x < XT; x++)
 #pragma unroll
-                for (int r = 0; r < 16; r++) acc[x][r] += red[(size_t) g * WN * XT * 1024 + x * 1024 + r * 64];
+            for (int r = 0; r < 16; r++) {
+                Sum v[KG];
+                v[0] = acc[x][r];
+#pragma unroll
+                for (int g = 1; g < KG; g++) v[g] = red[(size_t) (g - 1) * RS + x * 1024 + r * 64];
+#pragma unroll
+                for (int o = 1; o < KG; o <<= 1)
+#pragma unroll
+                    for (int g = 0; g < KG; g += 2 * o) v[g] += v[g + o];
+                acc[x][r] = v[0];
+            }
     }
     if (n >= a.N) return;
 #pragma unroll
@@ -413,7 +422,8 @@ __global__ __launch_bounds__(64 * WN * KG, 2) void k_gemm_kq(const KqArgs a) {
             const int m = m0 + x * 32 + 8 * (r >> 2) + 4 * lk + (r & 3);
             if (m >= a.M) continue;
             const size_t o = (size_t) m * a.ldy + n;
-            a.y[o] = a.res ? acc[x][r] + a.res[o] : acc[x][r];
+            const float v = (float) acc[x][r];
+            a.y[o] = a.res ? v + a.res[o] : v;
         }
 }
 
@@ -442,19 +452,26 @@ void run_kq(const void * wv, int64_t N, int64_t K, const void * act, int64_t M, 
     a.raw_sb = raw_sb;
     const auto tiles = [&](int64_t tm, int64_t tn) { return ((M + tm - 1) / tm) * ((N + tn - 1) / tn); };
     // 64 x 128 tiles where they fill the chip; else 64 x 64 in two K groups; where 32 x 32 tiles are few, those in
-    // eight. Each K group needs super-blocks: one, and groups only wait; two, and eight groups do the work of two;
-    // below eight, 64 x 128 tiles are worth half as many of them and 32 x 32 tiles only one per CU. Kernel times, Q4_K, us for
-    // 64 x 128 / 64 x 64 / 32 x 32 tiles: 512 x 4096 x 14336 115 / 92 / 164; 128 x 4096 x 4096 32 / 21 / 19; 128 x 4096 x 256
-    // 6.2 / 7.1 / 11.2; 256 x 2048 x 512 8.2 / 7.3 / 11.7; 65 x 4096 x 1024 11.3 / 8.9 / 11.3; 33 x 4096 x 1024 10.9 / 8.3 / 6.9.
-    // 765 shapes of 9 to 2048 rows, 96 to 128256 columns and K 256 to 14336: within 1 % of the best of the three on average
-    // for each type, at most 17 % off it.
+    // eight. Each K group needs super-blocks: one or two, and most groups only wait; below eight, 64 x 128 tiles are worth
+    // half as many of them and 32 x 32 tiles only one per CU. Kernel times, Q4_K, us for 64 x 128 / 64 x 64 / 32 x 32 tiles:
+    // 512 x 4096 x 14336 115 / 92 / 164; 128 x 4096 x 4096 32 / 21 / 19; 128 x 4096 x 256 6.2 / 7.1 / 11.2; 256 x 2048 x 512
+    // 8.2 / 7.3 / 11.7; 65 x 4096 x 1024 11.3 / 8.9 / 11.3; 33 x 4096 x 1024 10.9 / 8.3 / 6.9.
+    // The groups' sums must be no further from 64 bits than one f32 chain over K. Eight sums of a super-block or two
+    // added one by one were 1.12 times as far (Q6_K, K 2048); in pairs they are not from eight super-blocks on, below that the
+    // 32 x 32 tiles sum in f64 (5-10 % of their time), and 64 x 64 tiles start at four.
     if constexpr (RAW) {
         k_gemm_kq<TYPE, 2, 4, 1, RAW><<<(unsigned) tiles(64, 128), 256, 0, s>>>(a);
     } else {
         const int64_t cus = cu_count();
-        if (a.nsb == 1 || tiles(64, 128) > (a.nsb < 8 ? cus / 2 : cus)) k_gemm_kq<TYPE, 2, 4, 1, RAW><<<(unsigned) tiles(64, 128), 256, 0, s>>>(a);
-        else if (a.nsb == 2 || tiles(32, 32) > (a.nsb < 8 ? cus : 2 * cus)) k_gemm_kq<TYPE, 2, 2, 2, RAW><<<(unsigned) tiles(64, 64), 256, 0, s>>>(a);
-        else k_gemm_kq<TYPE, 1, 1, 8, RAW><<<(unsigned) tiles(32, 32), 512, 0, s>>>(a);
+        const bool few = a.nsb < 8;
+        if (a.nsb > 2 && tiles(64, 128) <= (few ? cus / 2 : cus) && tiles(32, 32) <= (few ? cus : 2 * cus)) {
+            if (few) k_gemm_kq<TYPE, 1, 1, 8, RAW, double><<<(unsigned) tiles(32, 32), 512, 0, s>>>(a);
+            else k_gemm_kq<TYPE, 1, 1, 8, RAW><<<(unsigned) tiles(32, 32), 512, 0, s>>>(a);
+        } else if (a.nsb > 3 && tiles(64, 128) <= (few ? cus / 2 : cus)) {
+            k_gemm_kq<TYPE, 2, 2, 2, RAW><<<(unsigned) tiles(64, 64), 256, 0, s>>>(a);
+        } else {
+            k_gemm_kq<TYPE, 2, 4, 1, RAW><<<(unsigned) tiles(64, 128), 256, 0, s>>>(a);
+        }
     }
 }
 

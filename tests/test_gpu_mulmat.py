@@ -324,6 +324,38 @@ def test_gemm_kquant_k_groups(gops, orc, t, M, N, K):
     assert orc.parity(y, orc.mul_mat(raw, t, x, K)) < 1e-5
 
 
+@pytest.mark.parametrize("t", ["q4_K", "q6_K"])
+@pytest.mark.parametrize("M,N,K", [(67, 1563, 2048), (39, 1280, 2304), (200, 1000, 1024), (70, 900, 512), (40, 700, 768),
+                                   (500, 1000, 768), (300, 2000, 1024), (33, 2000, 4096), (40, 900, 1792)])
+def test_gemm_kquant_precision(gops, orc, t, M, N, K):
+    """The K groups' f32 sums are no further from float64 than one chain of multiply-adds over the super-blocks (3 %: how
+    far the ratio moves with the inputs). The super-blocks' integers are exact (gemm_block_isums)."""
+    raw, qw = _weight(gops, orc, t, N, K, 47)
+    x = orc.normal((M, K), seed=48)
+    act = gops.quantize_act(t, torch.from_numpy(x).cuda())
+    y = to_np(gops.mul_mat_q(qw, act, M)).astype(np.float64)
+    nsb = K // 256
+    blocks = raw.reshape(N, nsb, -1)
+    f16 = lambda b: np.ascontiguousarray(b).view(np.float16)[..., 0].astype(np.float64)  # noqa: E731
+    d, dm = (f16(blocks[:, :, 208:210]), None) if t == "q6_K" else (f16(blocks[:, :, 0:2]), f16(blocks[:, :, 2:4]))
+    xb = x.reshape(M, nsb, 256)
+    top = np.take_along_axis(xb, np.abs(xb).argmax(2)[..., None], 2)[..., 0]
+    dx = (np.float32(1) / (np.float32(-127) / top)).astype(np.float64)
+    exact, chain = np.zeros((M, N)), np.zeros((M, N))
+    f32 = lambda v: v.astype(np.float32).astype(np.float64)  # noqa: E731
+    for sb in range(nsb):
+        i = to_np(gops.gemm_block_isums(qw, act, M, sb)).astype(np.float64)
+        if dm is None:
+            part, v = d[None, :, sb] * i, f32(d[None, :, sb] * f32(i))
+        else:
+            part = d[None, :, sb] * i[:, :, 0] - dm[None, :, sb] * i[:, :, 1]
+            v = f32(f32(d[None, :, sb] * f32(i[:, :, 0])) - dm[None, :, sb] * i[:, :, 1])
+        exact += dx[:, None, sb] * part
+        chain = f32(chain + dx[:, None, sb] * v)
+    e, c = np.sqrt(np.sum((y - exact) ** 2)), np.sqrt(np.sum((chain - exact) ** 2))
+    assert e < 1.03 * c
+
+
 @pytest.mark.parametrize("t", ["q4_0", "q8_0"])
 @pytest.mark.parametrize("M,N,K", [(9, 31, 32), (33, 65, 96), (40, 200, 1056), (33, 6200, 160), (97, 16300, 288),
                                    (300, 9100, 160), (129, 24800, 96), (17, 90200, 96)])
