@@ -9,11 +9,11 @@
 // view of the first n_kv rows of a [Hkv][max_context][D] cache); mask [s][j] f16 (row stride
 // m_s); out [s][h][Dv] f32, ggml's ne = [Dv, H, Sq].
 //
-// Attention is HBM-bound by the K/V stream. Both kernels split the keys: grid = (split, KV head
+// Attention is HBM-bound by the K/V stream for few rows. The kernels split the keys: k_attn_split's grid = (split, KV head
 // [, query row]), each workgroup streams one contiguous slice of its KV head's rows once and
 // serves all G = H/Hkv query heads that share it. One query row (decode) runs k_attn_decode on the
-// matrix cores; several rows run k_attn_prompt (attn_prompt.hip); head sizes, masks and scales it does not
-// take run k_attn_split (D/8 lanes cover one 2*D-byte row; pass 1 forms the
+// matrix cores, up to 2048 keys k_attn_lanes; several rows run k_attn_prompt (attn_prompt.hip); a few short
+// rows (attn_few_rows) and head sizes, masks and scales it does not take run k_attn_split (D/8 lanes cover one 2*D-byte row; pass 1 forms the
 // scores with v_dot2_f32_f16 into LDS, pass 2 the slice's max and exp-sum, pass 3 P.V). A merge
 // (k_attn_merge, or the prologue of the GEMV that reads the attention row) combines the splits'
 // (max, sum, partial output) exactly as one online softmax would.

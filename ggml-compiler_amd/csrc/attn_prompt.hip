@@ -8,8 +8,9 @@
 //   - scores S^T[key][row] = K Q^T with v_mfma_f32_32x32x16_f16 (Q rounded to f16): lane (row, half lk)
 //     is left with keys 8 i + 4 lk + r of its row, so a row's softmax needs one exchange with lane ^ 32;
 //   - O^T[dim][row] += V^T P^T: P is used where the scores lie (the MFMA's k slots are those keys, V^T
-//     read in the same order), in two f16 parts, P and its remainder, scaled by 2^13 so that the
-//     parts keep 22 bits of every weight down to 2^-27 of the largest (f16 has no finer step there).
+//     read in the same order), scaled by 2^15, as NP f16 parts: its rounding, the remainder's rounding, ..
+//     Two parts hold 22 bits of a weight down to 2^-17 of 2^R below, three all 24 bits down to 2^-16; smaller
+//     weights to an absolute 2^-40 of 2^R (f16's finest step), the f32 sum's own rounding being 2^-24 of more.
 // The softmax runs in powers of two against an integer reference R >= the running maximum: raising
 // R rescales by an exact power of two and is rare, and splits with the same R merge without rounding.
 // Blocks that no row of the workgroup sees (mask all -inf: k_attn_mask_bits looks the mask over first; or
@@ -22,11 +23,12 @@
 // layout and go through the same merges.
 //
 // What bounds it: per 32 rows x 32 keys at D = 128, 24 MFMAs (8 for the scores, 16 for the two parts of
-// P V) of 32 clocks, about 210 VALU operations, and the latency of the LDS operands, which two
-// wavefronts per SIMD (256 registers) do not hide: the matrix cores are busy a third of the time. 32 / 8
+// P V) of 32 clocks, about 300 other VALU operations, and the latency of the LDS operands, which two
+// wavefronts per SIMD (256 registers) do not hide: the matrix cores are busy 28 % of the cycles. 32 / 8
 // heads x 128, 512 rows over 4096 keys, causal mask: 817 us with the per-row kernel (K / V read again for
-// every query row, dots on the VALU), 86 us so with the look at the mask and the merge (the kernel
-// 80); 2048 rows over 2048 keys: 1667 -> 124 us. Both kernels are 2.3e-7 off 64 bits at 4096 keys.
+// every query row, dots on the VALU), 92 us so with the look at the mask and the merge (the kernel
+// 86); 2048 rows over 2048 keys: 1661 -> 131 us. Off 64 bits at 4096 keys: 1.9e-7, the per-row
+// kernel 2.3e-7.
 #include "gcq_common.h"
 
 #include <algorithm>
@@ -44,8 +46,8 @@ typedef float v16f __attribute__((ext_vector_type(16)));
 
 constexpr int KB = 64;          // keys per block
 constexpr int VP = KB + 4;      // pitch of a V^T row (halves): 16 lanes' 8-byte reads in distinct banks
-// Up to these keys every block takes the mask: looking it over first costs a launch (129 rows x 256 keys, 14 / 2
-// heads of 64: 22.2 us with it, 18.9 without).
+// Up to these keys, or 64 rows of a KV head, every block takes the mask: looking it over first costs a launch (129 rows x 256
+// keys, 14 / 2 heads of 64: 22.2 us with it, 18.9 without; 2 rows x 32768 keys, 8 heads of 64: 27.9 us and 23.5 in k_attn_split).
 constexpr int kBitsKeys = 512;
 constexpr float kPScale = 32768.0f;  // P's scale
 
@@ -256,7 +258,7 @@ __global__ __launch_bounds__(64 * RW * KW, RW == 1 ? 1 : 2) void k_attn_prompt(c
         if (MODE == kMask && KW == 1 && some) load_mask(b);
         load(min(bn, b1 - 1));
         // Dots of D values: chains of two MFMAs, added in f32. A sum inside the MFMA is cut off, not rounded, against a
-        // growing accumulator (one chain of eight: 1.10 times the error of f32 dots, four chains 0.95).
+        // growing accumulator (one chain of eight: 1.10 times the error of f32 dots, chains of two 0.95).
         v16f S[KT];
         const _Float16 * kp = lds.k + (32 * (KW == 2 ? kw : 0) + lr) * KP + 8 * lk;
 #pragma unroll
@@ -529,7 +531,8 @@ void run_rows(const PromptArgs & a, int Hkv, int mode, int rg, hipStream_t s) {
 }  // namespace
 
 // (A mask needs rows of at least four values: launch_attn_prompt.) The scale's range: a dropped key's weight is
-// 2^(scale -inf), not 0 where the scale is 0, and a mask value is divided by the scale; k_attn_split takes the rest.
+// 2^(scale -inf), no 0 where the scale is 0, and near the ends of f32 scale2 or its products leave it; k_attn_split takes the
+// rest.
 bool attn_prompt_fits(int D, int Sq, int H, int Hkv, float scale) {
     return (D == 64 || D == 128) && Sq > 1 && H % Hkv == 0 && H / Hkv <= 8 && (int64_t) Sq * (H / Hkv) < INT32_MAX &&
            fabsf(scale) >= 0x1p-60f && fabsf(scale) <= 0x1p60f;
@@ -550,15 +553,15 @@ AttnPlan attn_plan_prompt(int Sq, int H, int Hkv, int n_kv) {
     return {(nblk + blocks - 1) / blocks, blocks * KB};
 }
 
-// Sq query rows over n_kv keys. mask: [Sq][m_s] f16 (added to the scaled scores; -inf drops a key), or null;
-// pos0 >= 0 (mask null): row s sees keys 0 .. pos0 + s. out [s][h][D] (one split), or null: partials
-// (part_o, part_ml) for a merge. bits: attn_prompt_bits bytes for a mask, else null.
 // Bytes of the mask's block bits.
 size_t attn_prompt_bits(int Sq, int H, int Hkv, int n_kv) {
     const int64_t rows = (int64_t) Sq * (H / Hkv), tile = 32 * row_groups(rows);
     return align256((size_t) ((rows + tile - 1) / tile) * ((n_kv + 32 * KB - 1) / (32 * KB)) * sizeof(uint2));
 }
 
+// Sq query rows over n_kv keys. mask: [Sq][m_s] f16 (added to the scaled scores; -inf drops a key), or null;
+// pos0 >= 0 (mask null): row s sees keys 0 .. pos0 + s. out [s][h][D] (one split), or null: partials
+// (part_o, part_ml) for a merge. bits: attn_prompt_bits bytes for a mask, else null.
 void launch_attn_prompt(const float * q, int64_t q_h, int64_t q_s, const void * k, int64_t k_h, int64_t k_j,
                         const void * v, int64_t v_h, int64_t v_j, const void * mask, int64_t m_s, int pos0, int D, int Sq,
                         int H, int Hkv, int n_kv, float scale, float * out, float * part_o, float2 * part_ml,

@@ -6,11 +6,13 @@
 //  rmsnorm_q8   ggml_rms_norm + ggml_mul (norm weight) + the Q8_0 conversion the next mul_mat
 //               makes of its src1. The f32 values are those of k_rms_norm, and the codes those of
 //               k_act_q8_0 on them, bit for bit.
-//  rope_kv      ggml_rope_ext (NEOX) on the q and k heads of a fused QKV row, q in place, and the
-//               ggml_set_rows of the roped k and of v into an f16 KV cache.
+//  rope_kv      ggml_rope_ext (NEOX) on the q and k heads of a fused QKV row, q in place or from the
+//               packed row order into another buffer, and the ggml_set_rows of the roped k and of v into an
+//               f16 KV cache.
 //  swiglu_q8    ggml_swiglu_split + the Q8_0 conversion of the down projection's src1.
 //  merge_q8     the split-K attention merge + the Q8_0 conversion of the output projection's src1.
-//  causal_mask  the additive f16 mask of ggml_compiler/llm.py:355-358 for a prompt chunk.
+//  causal_mask  the additive f16 mask of ggml_compiler/llm.py:355-358 for a prompt of one row (longer ones are causal
+//               by position, attn_prompt.hip).
 //  step_end     ggml_argmax of the logits plus the generate loop's bookkeeping
 //               (runtime/src/ggml_compiler_rt.cpp:402-439): the next token, position and KV length.
 #include "gcq_common.h"
@@ -179,12 +181,10 @@ __global__ void k_embed_rope(int type, const uint8_t * __restrict__ tab, int64_t
     }
 }
 
-// mask[s][j] = 0 for j <= pos0 + s, -inf after (f16), j < n_kv.
-__global__ void k_causal_mask(uint16_t * __restrict__ mask, int S, int n_kv, int pos0) {
-    const int64_t t = (int64_t) blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= (int64_t) S * n_kv) return;
-    const int s = (int) (t / n_kv), j = (int) (t % n_kv);
-    mask[t] = j <= pos0 + s ? (uint16_t) 0 : (uint16_t) 0xfc00;
+// mask[j] = 0 for j <= pos, -inf after (f16), j < n_kv: the mask of one row.
+__global__ void k_causal_mask(uint16_t * __restrict__ mask, int n_kv, int pos) {
+    const int j = blockIdx.x * blockDim.x + threadIdx.x;
+    if (j < n_kv) mask[j] = j <= pos ? (uint16_t) 0 : (uint16_t) 0xfc00;
 }
 
 // argmax of the logits (first index of the maximum) and the generate loop's step: record the
@@ -317,8 +317,8 @@ void launch_embed_rope(int type, const void * tab, int64_t nrows, int64_t D, con
     check_launch("embed_rope");
 }
 
-void launch_causal_mask(void * mask, int S, int n_kv, int pos0, hipStream_t s) {
-    k_causal_mask<<<nblk((int64_t) S * n_kv, 256), 256, 0, s>>>((uint16_t *) mask, S, n_kv, pos0);
+void launch_causal_mask(void * mask, int n_kv, int pos, hipStream_t s) {
+    k_causal_mask<<<nblk(n_kv, 256), 256, 0, s>>>((uint16_t *) mask, n_kv, pos);
     check_launch("causal_mask");
 }
 

@@ -28,8 +28,9 @@
 // lane (column, k half) reads its column's 16-byte pieces and expands them to hi and lo codes right
 // where the MFMA takes them, its column's header (scales, mins, d) in its own registers.
 //
-// What bounds it: the VALU's issue (about 190 operations per wavefront and half super-block beside 16
-// MFMAs: the expansion, then 5 operations per output and super-block). Measured, the GEMM alone
+// What bounds it: the VALU's issue (about 200 operations per wavefront and half super-block beside 17
+// MFMAs: the expansion, then 5 operations per output and super-block; the matrix cores are busy 38 % of the
+// cycles at two wavefronts per SIMD). Measured, the GEMM alone
 // at Q4_K 1999 x 14336 x 4096: 435 us with the sub-block scales applied on the VALU (an integer
 // multiply-add per output and 32 values), 340 us as here; 33 x 4096 x 14336 (KG = 8): 133 -> 21 us.
 #include "gcq_common.h"

@@ -56,7 +56,7 @@ void launch_attn_prompt(const float * q, int64_t q_h, int64_t q_s, const void * 
                         const AttnPlan & p, void * bits, hipStream_t s);
 void launch_merge_q8(const float * part_o, const float2 * part_ml, int nsplit, int Sq, int H, int D, float * out,
                      void * act, hipStream_t s);
-void launch_causal_mask(void * mask, int S, int n_kv, int pos0, hipStream_t s);
+void launch_causal_mask(void * mask, int n_kv, int pos, hipStream_t s);
 void launch_move_rows(const void * src, void * dst, const int32_t * map, int64_t rows, int64_t row_bytes, bool scatter,
                       hipStream_t s);
 AttnPlan attn_plan_decode(int D, int H, int G, int max_ctx, int max_split);
@@ -565,7 +565,7 @@ struct Llama {
             check_hip(hipMemcpyAsync(positions.p, p.data(), n * 4, hipMemcpyHostToDevice, stream), "positions");
             check_hip(hipMemcpyAsync(xs, x_in, row_bytes, hipMemcpyHostToDevice, stream), "x");
             const int n_kv = pos0 + n;
-            if (n == 1) launch_causal_mask(mask.p, n, n_kv, pos0, stream);
+            if (n == 1) launch_causal_mask(mask.p, n_kv, pos0, stream);
             const AttnPlan plan = prompt_plan(n, n_kv);
             for (int l = first; l < first + count; l++)
                 prompt_layer(l, n, positions.as<int32_t>(), n_kv, nullptr, mask.p, plan,
@@ -585,7 +585,7 @@ struct Llama {
             std::memcpy(host_tokens.p, tokens + i, (size_t) S * 4);  // the last chunk has been waited for
             launch_prompt_in(host_tokens.as<int32_t>(), tok_in.as<int32_t>(), positions.as<int32_t>(), pos, S, stream);
             const int n_kv = pos + S;
-            if (S == 1) launch_causal_mask(mask.p, S, n_kv, pos, stream);
+            if (S == 1) launch_causal_mask(mask.p, n_kv, pos, stream);
             forward(S, tok_in.as<int32_t>(), positions.as<int32_t>(), n_kv, nullptr, mask.p, prompt_plan(S, n_kv));
             const bool out = logits_host && i + S == n;
             if (out) results_out(true);

@@ -98,8 +98,8 @@ __device__ __forceinline__ float code(float v) {
 // The K-quant encoders run a thread per sub-block, its 32 (16) values, weights and codes in
 // registers, every sum in the reference's order; the 8 (16) lanes of a super-block then exchange
 // scales and codes. What bounds them is the VALU: 21 candidates of 32 values, 17 operations each
-// (Q4_K). 4096 x 14336 values: Q4_K 5716 -> 530 us, Q5_K 4763 -> 410, Q6_K 482 -> 280 against a thread per
-// super-block with its arrays in scratch memory. The 146 registers leave three wavefronts per SIMD;
+// (Q4_K; 13668 instructions per wavefront, 3.4 issued per CU and ns). 4096 x 14336 values: Q4_K 5703 -> 452 us,
+// Q5_K 4774 -> 367, Q6_K 466 -> 260 against a thread per super-block with its arrays in scratch memory. The 146 registers leave three wavefronts per SIMD;
 // held to 128 for a fourth it spills: 590-720 us.
 
 // ggml make_qkx2_quants(32, NMAX, x, w, L, &min, Laux, rmin, 0.1, NSTEP, false): weighted
