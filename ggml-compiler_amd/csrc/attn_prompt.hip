@@ -538,14 +538,17 @@ bool attn_prompt_fits(int D, int Sq, int H, int Hkv, float scale) {
            fabsf(scale) >= 0x1p-60f && fabsf(scale) <= 0x1p60f;
 }
 
-// Key splits: about 512 workgroups in all (two per CU), each split of at least two key blocks, or one where that makes
-// few splits to merge (8; 16 for up to 256 output rows): 33 rows over 300 keys 23.0 us in two splits of three blocks, 16.1 in
-// five of one. No more for a smaller n_kv, so a bound for every KV length up to n_kv.
+// Key splits: about 512 workgroups in all (two per CU), each split of at least two key blocks, or one where the merge
+// stays small (16 splits for up to 256 output rows, 8 for up to 2048): 33 rows of 32 heads over 300 keys 23.0 us in two splits
+// of three blocks, 16.1 in five of one; 129 rows over 512 keys 18.5 in four of two, 24.4 in eight of one. No more for a smaller
+// n_kv, so a bound for every KV length up to n_kv.
 int attn_prompt_max_split(int Sq, int H, int Hkv, int n_kv) {
     const int64_t rows = (int64_t) Sq * (H / Hkv), tile = 32 * row_groups(rows);
     const int64_t wgs = (rows + tile - 1) / tile * Hkv;
     const int nblk = (n_kv + KB - 1) / KB;
-    return (int) std::max<int64_t>(1, std::min<int64_t>({512 / wgs, std::max(std::min(nblk, (int64_t) Sq * H <= 256 ? 16 : 8), nblk / 2), 64}));
+    const int64_t out = (int64_t) Sq * H;
+    const int singles = std::min(nblk, out <= 256 ? 16 : out <= 2048 ? 8 : 1);
+    return (int) std::max<int64_t>(1, std::min<int64_t>({512 / wgs, std::max(singles, nblk / 2), 64}));
 }
 AttnPlan attn_plan_prompt(int Sq, int H, int Hkv, int n_kv) {
     const int nblk = (n_kv + KB - 1) / KB, most = attn_prompt_max_split(Sq, H, Hkv, n_kv);
